@@ -309,6 +309,8 @@ Context::~Context()
     for (MultiTables &t : mtab)
         for (int h = 0; h < 2; ++h)
             if (t.tab[h]) (void)hipFree(t.tab[h]);
+    for (int h = 0; h < 2; ++h)
+        if (blk.tab[h]) (void)hipFree(blk.tab[h]);
     if (pinned) (void)hipHostFree(pinned);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -551,6 +553,7 @@ static int create_impl(const axs_params *p, int n_members, const int *Ns, axs_ct
         c->tune.depth = 1;
         c->tune.flags &= ~(kTuneWG512 | kTuneWG1024);
     }
+    c->tune_default = c->tune;
     (void)rc;
     *out = h;
     return AXS_OK;
@@ -783,12 +786,16 @@ int axs_step(axs_ctx *ctx, int64_t nsteps)
             return AXS_ERR_STATE;
         }
     if (nsteps == 0) return AXS_OK;
-    AXS_TRY(prepare_batch(c));
+    const int blk = block2d_depth(c);
+    if (blk > 0)
+        AXS_TRY(prepare_block2d(c));
+    else
+        AXS_TRY(prepare_batch(c));
     const double dt = (double)c->p.time_step;
     // the spectral step's rocFFT calls stay out of graph capture
     const bool graph = (c->tune.flags & kTuneGraph) && nsteps > 1 &&
                        c->p.laplacian == AXS_LAPLACIAN_STENCIL;
-    AXS_TRY(prepare_passes(c, nsteps));
+    if (blk == 0) AXS_TRY(prepare_passes(c, nsteps));
     const double tau0 = c->tau;
     const int cur0 = c->cur;
     hipGraph_t g = nullptr;
@@ -804,7 +811,7 @@ int axs_step(axs_ctx *ctx, int64_t nsteps)
         double tau_next = c->tau + dt;                    // s_integrate.cpp:317
         StepScalars s = make_scalars(c->p, tau_next);
         const int64_t left = nsteps - n;
-        const int d = next_pass_depth(c, left);
+        const int d = (blk > 0) ? (int)std::min<int64_t>(left, blk) : next_pass_depth(c, left);
         if (!graph && c->step_fail_after >= 0 && launches >= c->step_fail_after) {
             set_error("axs_step: failure point after %d launches (AXS_STEP_FAIL_AFTER)",
                       launches);
@@ -818,7 +825,7 @@ int axs_step(axs_ctx *ctx, int64_t nsteps)
                 t = t + dt;                               // the same sequence of sums
                 ss[l] = make_scalars(c->p, t);
             }
-            rc = launch_multi_steps(c, ss, d);
+            rc = (blk > 0) ? launch_block2d(c, ss, d) : launch_multi_steps(c, ss, d);
             if (rc == AXS_OK) {
                 c->tau = t;
                 ++launches;
@@ -1096,6 +1103,7 @@ int axs_set_kernel_config(axs_ctx *ctx, const axs_kernel_config *cfg)
     c->tune.ci64 = cfg->chunk;
     c->tune.depth = depth;
     c->tune.flags = cfg->flags;
+    c->tune.configured = true;
     return AXS_OK;
 }
 

@@ -138,6 +138,9 @@ struct Tune {
                        // one-step kernels for the 7/5-point stencil)
     int rtb = 0;       // rows per work-item of the multi-step kernel, 0 = by side
     int flags = kTunePrefetch | kTuneNT;
+    // a launch shape set by the caller or chosen by the tuner: the
+    // automatic choices of kernel (block2d_depth) no longer apply
+    bool configured = false;
 };
 
 constexpr int kTuneGraph = 8;      // capture the step loop in a HIP graph
@@ -153,6 +156,7 @@ struct Context {
     int cur = 0;                  // ping-pong index holding the current state
     double tau = 1.0;             // physics.cpp:32
     Tune tune;
+    Tune tune_default;            // the shape the context was created with
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t stage_ev[2] = {nullptr, nullptr};   // copy_to_host chunk completions
@@ -220,6 +224,9 @@ struct Context {
         uint32_t items = 0;
     };
     MultiTables mtab[kMaxDepth + 1];
+    // blocks of the small 2D lattices' kernel; one lattice's entry by value
+    MultiTables blk;
+    BatchMember blk_one[2] = {};
     // string finder results of the last call (ballot words, block counts,
     // offsets), reused while the member's state is unchanged
     void *strbuf = nullptr;
@@ -300,6 +307,11 @@ int prepare_march2d_items(Context *c, int D);
 int launch_march2d(Context *c, int src, const StepScalars *s, int depth);
 // higher-order stencils (radius 2-4), 2D (axs_march2d_hi.hip)
 int launch_march2d_high_order(Context *c, int src, const StepScalars *s, int depth, bool pf);
+// small 2D lattices (axs_block2d.hip): most steps of one pass, or 0 where
+// the strip kernels run
+int block2d_depth(const Context *c);
+int prepare_block2d(Context *c);
+int launch_block2d(Context *c, const StepScalars *s, int d);
 // field-rescaled step with the spectral Laplacian, one member
 int run_spectral_step(Context *c, Member &m, int src, int dst, const StepScalars &s);
 // Laplacian of the current field (AXS_LAPLACIAN_*) into host arrays

@@ -20,22 +20,42 @@ bool march2d_depth_built(int D, int RAD, int prec)
     return D >= 1 && D <= ((prec == AXS_FP64) ? 2 : 4);
 }
 
-// rows per chunk for every member: the configured count if it divides N;
-// else the longest chunk of 128, 64 or 32 rows (fewer halo rows per chunk)
-// that still deals the chip about 8 waves per SIMD (FP32; 4 in FP64, whose
-// kernels hold more registers).  Measured: 128 for the 512-lattice ensemble
-// of sides 128..1024 and single lattices from 8192^2 on; 32 (FP32) and 64
-// (FP64) at 4096^2, 1.3-1.4x faster there than 128.
-static int pick_cap(const Context *c, int TI)
+// Rows per chunk, unless configured, by a cost model.  A wave marches chunk +
+// 2H rows (H = halo); w = waves per SIMD share its issue, and a wave alone
+// leaves a SIMD idle for the row's dependent chain and its loads.  A pass
+// takes about (w + b) (chunk + 2H), b = 3 in FP32 and 1 in FP64 (whose rows
+// fill the issue): fitted to chunks 8..128 at sides 720..2048 and 4096, where
+// it is within 10% of the best chunk measured.  It keeps 128 for the
+// 512-lattice ensemble and 32 (FP32) / 64 (FP64) at 4096^2; at 1000^2 it
+// takes 10-row chunks (FP64 depth 6: 46 -> 40 us a pass; FP64 second order,
+// depth 2: 35 -> 28 us; FP32 22 -> 16 us), where 32 rows left half the SIMDs
+// without a wave.
+static int pick_cap(const Context *c, int TI, int H)
 {
-    const uint64_t target = (uint64_t)c->num_cu * 4u * ((c->prec == AXS_FP32) ? 8u : 4u);
-    for (int cap = 128; cap > 32; cap >>= 1) {
-        uint64_t waves = 0;
+    const double simds = 4.0 * (c->num_cu > 0 ? c->num_cu : 1);
+    const double b = (c->prec == AXS_FP32) ? 3.0 : 1.0;
+    int best = 8;
+    double best_cost = 1e300;
+    for (int cap = 128; cap >= 8; cap >>= 1) {
+        double waves = 0.0;
         for (const Member &m : c->members)
-            waves += (uint64_t)((m.N + TI - 1) / TI) * (uint64_t)(m.N / divisor_below(m.N, cap));
-        if (waves >= target) return cap;
+            waves += (double)((m.N + TI - 1) / TI) * (double)((m.N + cap - 1) / cap);
+        const double cost = (waves / simds + b) * (double)(cap + 2 * H);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = cap;
+        }
     }
-    return 32;
+    return best;
+}
+
+// rows per chunk of a lattice of side N for a choice of `cap` rows: the
+// chunks are made equal to within a row (the last one is shorter where they
+// do not divide N)
+static int chunk_rows(int N, int cap)
+{
+    const int n = (N + cap - 1) / cap;
+    return (N + n - 1) / n;
 }
 
 int prepare_march2d_items(Context *c, int D)
@@ -46,7 +66,7 @@ int prepare_march2d_items(Context *c, int D)
     const int key = ((D * 10 + RAD) * 100 + 2) * 10000 + c->tune.ci32;
     if (key == mt.key && mt.tab[0]) return AXS_OK;
     const int TI = kW2 - 2 * D * RAD;
-    const int cap = pick_cap(c, TI);
+    const int cap = pick_cap(c, TI, D * RAD);
     std::vector<BatchMember> tab[2];
     uint32_t items = 0;
     for (const Member &m : c->members) {
@@ -57,8 +77,8 @@ int prepare_march2d_items(Context *c, int D)
         b.nTj = (m.N + TI - 1) / TI;       // strips
         b.nTk = 1;
         const int cfg = c->tune.ci32;      // rows per chunk
-        b.CI = (cfg > 0 && m.N % cfg == 0) ? cfg : divisor_below(m.N, cap);
-        items += (uint32_t)b.nTj * (uint32_t)(m.N / b.CI);
+        b.CI = (cfg > 0 && m.N % cfg == 0) ? cfg : chunk_rows(m.N, cap);
+        items += (uint32_t)b.nTj * (uint32_t)((m.N + b.CI - 1) / b.CI);
         for (int h = 0; h < 2; ++h) {
             for (int a = 0; a < 3; ++a) {
                 b.in[a] = m.state[h][a];

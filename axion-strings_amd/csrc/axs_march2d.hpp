@@ -52,7 +52,7 @@ constexpr int strip_unroll()
 }
 
 template <class Tr, int D, int RAD, bool PF>
-__device__ __forceinline__ void march2d_strip(const int N, const int CJ, const int ti,
+__device__ __forceinline__ void march2d_strip(const int N, const int chunk, const int ti,
                                               const int ch, const typename Tr::In &in,
                                               const typename Tr::Out &out,
                                               const LevelScalars<typename Tr::Sc, D> &sc)
@@ -64,7 +64,8 @@ __device__ __forceinline__ void march2d_strip(const int N, const int CJ, const i
     constexpr int TI = kW2 - 2 * H;      // columns written
     static_assert(TI > 0, "strip shape");
     const int lane = threadIdx.x & 63;
-    const int i0 = ti * TI, j0 = ch * CJ;
+    const int i0 = ti * TI, j0 = ch * chunk;
+    const int CJ = (N - j0 < chunk) ? N - j0 : chunk;      // the last chunk may be shorter
     int ii = i0 - H + lane;              // -H <= ii < 2N for N >= 64
     ii = (ii < 0) ? ii + N : ((ii >= N) ? ii - N : ii);
     const bool colout = lane >= H && lane < kW2 - H && (i0 + lane - H) < N;

@@ -55,7 +55,8 @@ void load_file_cache()
     if (!f) return;
     char line[1024];
     while (fgets(line, sizeof line, f)) {
-        // key | kernel rj32 rj64 ci32 ci64 flags | ms
+        // key | kernel rj32 rj64 ci32 ci64 flags depth rows [configured] | ms
+        // (files without the ninth number hold configured shapes only)
         char *bar1 = strchr(line, '|');
         if (!bar1) continue;
         char *bar2 = strchr(bar1 + 1, '|');
@@ -64,10 +65,13 @@ void load_file_cache()
         while (!key.empty() && key.back() == ' ') key.pop_back();
         Tune t;
         double ms = 0;
-        if (sscanf(bar1 + 1, "%d %d %d %d %d %d %d %d", &t.kernel, &t.rj32, &t.rj64, &t.ci32,
-                   &t.ci64, &t.flags, &t.depth, &t.rtb) == 8 &&
-            sscanf(bar2 + 1, "%lf", &ms) == 1)
+        int conf = 1;
+        if (sscanf(bar1 + 1, "%d %d %d %d %d %d %d %d %d", &t.kernel, &t.rj32, &t.rj64, &t.ci32,
+                   &t.ci64, &t.flags, &t.depth, &t.rtb, &conf) >= 8 &&
+            sscanf(bar2 + 1, "%lf", &ms) == 1) {
+            t.configured = conf != 0;
             g_tune_cache[key] = {t, ms};
+        }
     }
     fclose(f);
 }
@@ -78,18 +82,22 @@ void append_file_cache(const std::string &key, const Tune &t, double ms)
     if (!path || !*path) return;
     FILE *f = fopen(path, "a");
     if (!f) return;
-    fprintf(f, "%s | %d %d %d %d %d %d %d %d | %.6f\n", key.c_str(), t.kernel, t.rj32, t.rj64,
-            t.ci32, t.ci64, t.flags, t.depth, t.rtb, ms);
+    fprintf(f, "%s | %d %d %d %d %d %d %d %d %d | %.6f\n", key.c_str(), t.kernel, t.rj32, t.rj64,
+            t.ci32, t.ci64, t.flags, t.depth, t.rtb, t.configured ? 1 : 0, ms);
     fclose(f);
 }
 
 // time `trials` steps of the current configuration without changing state
 int time_trial(Context *c, int trials, double *ms)
 {
-    AXS_TRY(prepare_batch(c));
+    const int blk = block2d_depth(c);     // the automatic shape of a small 2D lattice
+    if (blk > 0)
+        AXS_TRY(prepare_block2d(c));
+    else
+        AXS_TRY(prepare_batch(c));
     const int cur0 = c->cur;
     const double dt = (double)c->p.time_step;
-    const int depth = multi_depth(c);     // 0: the one-step kernels
+    const int depth = (blk > 0) ? blk : multi_depth(c);     // 0: the one-step kernels
     StepScalars ss[kMaxDepth];
     double t = c->tau;
     for (int l = 0; l < kMaxDepth; ++l) {
@@ -98,7 +106,10 @@ int time_trial(Context *c, int trials, double *ms)
     }
     const StepScalars &s = ss[0];
     // one trial = one launch of one or several steps
-    auto one = [&]() { return depth >= 1 ? launch_multi_steps(c, ss, depth) : launch_step(c, s); };
+    auto one = [&]() {
+        if (blk > 0) return launch_block2d(c, ss, blk);
+        return depth >= 1 ? launch_multi_steps(c, ss, depth) : launch_step(c, s);
+    };
     AXS_TRY(one());                             // warm-up (code objects, caches)
     c->cur = cur0;
     const bool graph = (c->tune.flags & kTuneGraph) != 0;
@@ -267,14 +278,23 @@ int run_autotune(Context *c, int trials, double *best_ms)
                     cands.push_back(u);
                 }
     }
+    for (Tune &t : cands) t.configured = true;
     const Tune saved = c->tune;
+    // the block kernel of small 2D lattices runs in the context's own shape,
+    // reported as the shape that runs without it
+    c->tune = c->tune_default;
+    if (block2d_depth(c) > 0) {
+        Tune u = c->tune_default;
+        u.kernel = strips_ok ? AXS_KERNEL_MARCH : AXS_KERNEL_SIMPLE;
+        cands.push_back(u);
+    }
     Tune best = saved;
     double best_t = 1e300;
     for (const Tune &t : cands) {
         c->tune = t;
-        if (t.kernel == AXS_KERNEL_MARCH && (t.depth >= 2 || RAD > 1)) {
+        if (t.configured && t.kernel == AXS_KERNEL_MARCH && (t.depth >= 2 || RAD > 1)) {
             if (multi_depth(c) != t.depth) continue;
-        } else if (t.kernel == AXS_KERNEL_MARCH) {
+        } else if (t.configured && t.kernel == AXS_KERNEL_MARCH) {
             bool ok = true;
             for (const Member &m : c->members) ok = ok && march3d_supported(c, m.N);
             if (!ok) continue;

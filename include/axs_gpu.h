@@ -285,7 +285,9 @@ typedef struct axs_kernel_config {
                      depth + 1 where that depth is built (3D FP32, depth
                      4), else end with shallower multi-step passes where
                      built, else with one-step launches; every split gives
-                     the same bits.                                         */
+                     the same bits.  Small 2D lattices and sides below 64
+                     run up to six steps per pass on a kernel of their own,
+                     with the same bits, until a configuration is set.      */
     int flags;    /* AXS_MARCH_* bits                                       */
 } axs_kernel_config;
 
