@@ -312,6 +312,7 @@ Context::~Context()
     for (int h = 0; h < 2; ++h)
         if (blk.tab[h]) (void)hipFree(blk.tab[h]);
     if (pinned) (void)hipHostFree(pinned);
+    if (mail) (void)hipHostFree(mail);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     for (int h = 0; h < 2; ++h)
@@ -483,6 +484,11 @@ static int create_impl(const axs_params *p, int n_members, const int *Ns, axs_ct
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
         set_error("stream/event creation failed");
         return fail(AXS_ERR_HIP);
+    }
+    if (hipHostMalloc(&c->mail, std::max<size_t>(4096, (size_t)n_members * 16),
+                      hipHostMallocDefault) != hipSuccess) {
+        set_error("pinned result buffer failed");
+        return fail(AXS_ERR_OUT_OF_MEMORY);
     }
     c->members.resize(n_members);
     for (int r = 0; r < n_members; ++r) {

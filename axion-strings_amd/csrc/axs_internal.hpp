@@ -179,6 +179,9 @@ struct Context {
     // the compaction's counts survive its growth)
     void *listbuf = nullptr;
     size_t listbuf_bytes = 0;
+    // pinned host memory that kernels write small results to (counts, sums),
+    // 4 KiB or two counters per member: read after a stream synchronisation
+    void *mail = nullptr;
     // pinned host staging
     void *pinned = nullptr;
     size_t pinned_bytes = 0;

@@ -563,7 +563,9 @@ static int sample_sums(Context *c, Member &m, double out[kSampQ], const Workspac
     void *wsp = nullptr;
     AXS_TRY(workspace_for(c, ws, part_b + kSampQ * sizeof(double), &wsp));
     Kahan *part = (Kahan *)wsp;
-    double *dout = (double *)((char *)wsp + part_b);
+    // the folded sums go straight to the context's pinned mailbox; with a
+    // caller's workspace, to the workspace and then to the host
+    double *dout = ws ? (double *)((char *)wsp + part_b) : (double *)c->mail;
     const double lam = (double)c->p.lambda, T0 = (double)c->p.T_initial;
     const double tau2 = c->tau * c->tau, T03 = (T0 * T0) / 3.0, lam_4tau2 = lam / (4.0 * tau2);
     const bool uni = plane % 64 == 0;       // every wave's columns share their slices
@@ -583,9 +585,11 @@ static int sample_sums(Context *c, Member &m, double out[kSampQ], const Workspac
     }
     hipLaunchKernelGGL(fold_kernel, dim3(kSampQ), dim3(256), 0, c->stream, part, nb, kSampQ, dout);
     AXS_HIP_TRY(hipGetLastError());
-    AXS_HIP_TRY(hipMemcpyAsync(m.samp, dout, kSampQ * sizeof(double), hipMemcpyDeviceToHost,
-                               c->stream));
+    if (ws)
+        AXS_HIP_TRY(hipMemcpyAsync(m.samp, dout, kSampQ * sizeof(double), hipMemcpyDeviceToHost,
+                                   c->stream));
     AXS_HIP_TRY(hipStreamSynchronize(c->stream));
+    if (!ws) std::copy(dout, dout + kSampQ, m.samp);
     m.samp_valid = true;
     m.samp_version = m.version;
     m.samp_tau = c->tau;

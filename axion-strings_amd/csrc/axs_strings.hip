@@ -7,18 +7,19 @@
 // is always in ascending site order (the single-thread order), which also
 // fixes the 2D core count of s_run.cpp:101-109.
 //
-// Each site's angle (atan2(phi1, phi2) + pi) / (2 pi) is computed in FP64
-// once -- the reference's axion array (s_run.cpp:92-94) scaled as in
-// string_finding.cpp:14-16 -- rather than once per plaquette corner, and
-// the plaquette test leaves one 64-bit ballot word (a bitmask of flagged
-// sites) per 64 sites in site order.  3D: one pass over phi
-// (strings_march_kernel) keeps the angles of two planes of a tile in LDS,
-// then a small kernel counts the flags per block.  2D: pass 0 writes the
-// angles to a scratch array, pass 1 evaluates the plaquettes from it and
-// counts.  Then one work-group scans the block counts, and the writer
+// The plaquettes are tested on the scaled angles (atan2(phi1, phi2) + pi) /
+// (2 pi) -- the reference's axion array (s_run.cpp:92-94) scaled as in
+// string_finding.cpp:14-16 -- and the test leaves one 64-bit ballot word (a
+// bitmask of flagged sites) per 64 sites in site order, from one pass over
+// phi that screens with FP32 angles and decides the rest in FP64 (below).
+// 3D: strings_march_kernel keeps the angles of two planes of a tile in LDS;
+// 2D: strings2d_block keeps those of two rows in registers.  A count reads
+// the words; a coordinate list scans the flags per block, and the writer
 // re-reads the ballot words and writes the coordinates at their ordered
 // positions.  The search is skipped when the same member's unchanged state
 // was searched by the previous call.
+#include <string.h>
+
 #include <algorithm>
 
 #include "axs_atan2.hpp"
@@ -55,31 +56,11 @@ __device__ __forceinline__ bool plaquettes3(double n0, double ni, double nij, do
 // (string_finding.cpp:14-16).  scaled_angle: libm's atan2 rounded
 // correctly (the double-double evaluation of axs_atan2.hpp, bit for bit the
 // value the host build and the oracle give); it decides every flag that
-// depends on the last bits of an angle.  scaled_angle_fast: the device
-// library's atan2 (within a few ulp of it), for the 2D angle pass whose
-// plaquettes near the threshold are re-evaluated with scaled_angle.
+// depends on the last bits of an angle.
 __device__ __forceinline__ double scaled_angle(double a1, double a2)
 {
     double a = atan2_dd(a1, a2);
     return (a + M_PI) / (2 * M_PI);
-}
-
-__device__ __forceinline__ double scaled_angle_fast(double a1, double a2)
-{
-    double a = atan2(a1, a2);
-    return (a + M_PI) / (2 * M_PI);
-}
-
-template <class P>
-__global__ void __launch_bounds__(256)
-angle_kernel(uint32_t L, P phi, double *__restrict__ ang)
-{
-    uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < L) {
-        double a1, a2;
-        phi.get(m, a1, a2);
-        ang[m] = scaled_angle_fast(a1, a2);
-    }
 }
 
 // the reference's axion array (s_run.cpp:92-94): atan2(phi1, phi2) of every
@@ -96,120 +77,14 @@ axion_kernel(uint32_t L, P phi, double *__restrict__ out)
     }
 }
 
-// A three-edge sum from the fast angles (each within a few 1e-16 of the
-// correctly rounded one, so the sum within ~1e-15) decides the flag unless
-// it lies within this margin of the threshold; there the four corners'
-// angles are evaluated again with scaled_angle.
-constexpr double kAngleMargin = 0x1p-30;
-
-// 2D plaquette of site m (string_finding.cpp:17-20): corners (i,j),
-// (i+1,j), (i+1,j+1), (i,j+1), three edges
-template <class P>
-__device__ __forceinline__ bool plaquette_flag2(const double *__restrict__ ang, const P &phi,
-                                                uint32_t m, int N, double accept)
-{
-    const Site<2> s = decompose<2>(m, N);
-    const uint32_t q2 = shifted<2>(s, 0, 1, N);
-    const Site<2> s2 = decompose<2>(q2, N);
-    const uint32_t q3 = shifted<2>(s2, 1, 1, N);
-    const uint32_t q4 = shifted<2>(s, 1, 1, N);
-    double n1 = ang[m], n2 = ang[q2], n3 = ang[q3], n4 = ang[q4];
-    double sum = edge_theta(n1, n2) + edge_theta(n2, n3) + edge_theta(n3, n4);
-    if (fabs(sum - accept) < kAngleMargin) {
-        auto exact = [&](uint32_t q) {
-            double a1, a2;
-            phi.get(q, a1, a2);
-            return scaled_angle(a1, a2);
-        };
-        n1 = exact(m);
-        n2 = exact(q2);
-        n3 = exact(q3);
-        n4 = exact(q4);
-        sum = edge_theta(n1, n2) + edge_theta(n2, n3) + edge_theta(n3, n4);
-    }
-    return sum > accept;
-}
-
-// 2D plaquette test of block `blk` (kStrSpan sites) of one lattice from
-// its angles: one ballot word per wave and pass, the block's count in bcount
-template <class P>
-__device__ __forceinline__ void flag_block(int N, uint32_t L, const double *__restrict__ ang,
-                                           const P &phi, double accept,
-                                           uint64_t *__restrict__ words,
-                                           uint32_t *__restrict__ bcount, uint32_t blk)
-{
-    __shared__ uint32_t wave_tot[kStrBlock / 64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t total = 0;
-    uint32_t base = blk * (uint32_t)kStrSpan;
-    for (int it = 0; it < kStrIters; ++it) {
-        uint32_t m = base + it * kStrBlock + threadIdx.x;
-        bool f = (m < L) && plaquette_flag2(ang, phi, m, N, accept);
-        uint64_t w = __ballot(f);
-        uint32_t wi = (base + it * kStrBlock) / 64 + wave;
-        if (lane == 0 && (uint64_t)wi * 64 < L) words[wi] = w;
-        total += (uint32_t)__popcll(w);
-    }
-    if (lane == 0) wave_tot[wave] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t t = 0;
-        for (int w = 0; w < kStrBlock / 64; ++w) t += wave_tot[w];
-        bcount[blk] = t;
-    }
-}
-
-template <class P>
-__global__ void __launch_bounds__(kStrBlock)
-strings_flag_kernel(int N, uint32_t L, const double *__restrict__ ang, P phi, double accept,
-                    uint64_t *__restrict__ words, uint32_t *__restrict__ bcount)
-{
-    flag_block(N, L, ang, phi, accept, words, bcount, blockIdx.x);
-}
-
 // Ensemble-wide 2D finder: member r owns blocks [first_block, first_block +
 // ceil(L / kStrSpan)) of one concatenated index space (its words start at
-// word first_block * kStrSpan / 64, its angles at site_base); blk2mem maps
-// a block to its member.
+// word first_block * kStrSpan / 64); blk2mem maps a block to its member.
 struct StrMember {
     const void *phi[2];      // the field of either ping-pong half
-    uint64_t site_base;
     uint32_t L, first_block;
     int N, pad;
 };
-
-template <class P>
-__global__ void __launch_bounds__(kStrBlock)
-angle_batch_kernel(const StrMember *__restrict__ mem, const uint32_t *__restrict__ blk2mem,
-                   int half, double *__restrict__ ang)
-{
-    const StrMember M = mem[blk2mem[blockIdx.x]];
-    P phi;
-    phi.p = (decltype(phi.p))M.phi[half];
-    const uint32_t base = (blockIdx.x - M.first_block) * (uint32_t)kStrSpan;
-    for (int it = 0; it < kStrIters; ++it) {
-        const uint32_t m = base + it * kStrBlock + threadIdx.x;
-        if (m < M.L) {
-            double a1, a2;
-            phi.get(m, a1, a2);
-            ang[M.site_base + m] = scaled_angle_fast(a1, a2);
-        }
-    }
-}
-
-template <class P>
-__global__ void __launch_bounds__(kStrBlock)
-strings_flag_batch_kernel(const StrMember *__restrict__ mem, const uint32_t *__restrict__ blk2mem,
-                          int half, const double *__restrict__ ang, double accept,
-                          uint64_t *__restrict__ words, uint32_t *__restrict__ bcount)
-{
-    const StrMember M = mem[blk2mem[blockIdx.x]];
-    P phi;
-    phi.p = (decltype(phi.p))M.phi[half];
-    const size_t wbase = (size_t)M.first_block * (kStrSpan / 64);
-    flag_block(M.N, M.L, ang + M.site_base, phi, accept, words + wbase, bcount + M.first_block,
-               blockIdx.x - M.first_block);
-}
 
 // 3D finder in one pass over phi.  A work-group of kSfW waves owns a tile
 // of kSfTJ rows (j) x 64 columns (k) and marches along i over a chunk of
@@ -295,6 +170,120 @@ __device__ __forceinline__ float edge_theta_f(float a, float b)
 {
     float d = fabsf(b - a);
     return fminf(d, 1.0f - d);
+}
+
+// 2D plaquettes (string_finding.cpp:17-20: corners (i,j), (i+1,j), (i+1,j+1),
+// (i,j+1), three edges) of block `blk` (kStrSpan consecutive sites) of one
+// lattice, in one pass over phi with the 3D finder's screen: a wave takes 512
+// consecutive sites, evaluates the FP32 angles of each and of the site one row
+// up, and reads the right-hand corners from the next lane; the last lane's are
+// the next word's first.  Row ends, whose right neighbours lie N - 1 sites
+// back, evaluate theirs apart.  A sum within kSfMargin of the threshold, or
+// one that touches an untrusted angle (NaN), is decided by the four corners'
+// FP64 angles.  One ballot word per wave and word, the block's count in bcount
+// (null: not wanted).  Bound by the angles' vector issue (2.25 a site);
+// replaces an FP64 angle pass and a test pass over an 8 B/site array
+// (512-lattice FP32 ensemble, 178M sites: the whole count 1.42 -> 0.68 ms).
+template <class P>
+__device__ __forceinline__ void strings2d_block(int N, uint32_t L, const P &phi, double accept,
+                                                uint64_t *__restrict__ words,
+                                                uint32_t *__restrict__ bcount, uint32_t blk)
+{
+    __shared__ uint32_t wave_tot[kStrBlock / 64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n = (uint32_t)N;
+    const float hi = (float)accept + kSfMargin, lo = (float)accept - kSfMargin;
+    const uint32_t base = blk * (uint32_t)kStrSpan + (uint32_t)wave * (64 * kStrIters);
+    // the site one row up (periodic), and the FP32 angle of a site (NaN where
+    // it is not trusted); indexes past the lattice read its last site
+    auto up = [&](uint32_t m) { return m >= L - n ? m - (L - n) : m + n; };
+    auto angle = [&](uint32_t m) -> float {
+        float x, y;
+        const bool ok = phi_float(phi, m, x, y);
+        const float th = angle_turns_f(x, y);
+        return ok ? th : __builtin_nanf("");
+    };
+    auto at = [&](uint32_t m) { return m < L ? m : L - 1; };
+    float A[kStrIters + 1], B[kStrIters + 1];
+#pragma unroll
+    for (int t = 0; t < kStrIters; ++t) {
+        const uint32_t m = at(base + 64u * t + lane);
+        A[t] = angle(m);
+        B[t] = angle(up(m));
+    }
+    {
+        const uint32_t m = at(base + 64u * kStrIters);       // first lane's next word
+        A[kStrIters] = angle(m);
+        B[kStrIters] = angle(up(m));
+    }
+    uint32_t total = 0;
+#pragma unroll
+    for (int t = 0; t < kStrIters; ++t) {
+        const uint32_t m = base + 64u * t + lane;
+        const bool in = m < L;
+        float n2 = lane_next(A[t]), n3 = lane_next(B[t]);
+        const float e2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                             __builtin_bit_cast(int, A[t + 1])));
+        const float e3 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                             __builtin_bit_cast(int, B[t + 1])));
+        n2 = (lane == 63) ? e2 : n2;
+        n3 = (lane == 63) ? e3 : n3;
+        const bool edge = in && (m + 1) % n == 0;
+        const uint32_t q2 = edge ? m + 1 - n : m + 1;        // right neighbour
+        if (__ballot(edge)) {
+            if (edge) {
+                n2 = angle(q2);
+                n3 = angle(up(q2));
+            }
+        }
+        const float sum = edge_theta_f(A[t], n2) + edge_theta_f(n2, n3) + edge_theta_f(n3, B[t]);
+        bool f = in && sum > hi;
+        const bool undecided = in && !f && !(sum < lo);
+        if (__ballot(undecided)) {
+            if (undecided) {
+                auto exact = [&](uint32_t q) {
+                    double a1, a2;
+                    phi.get(q, a1, a2);
+                    return scaled_angle(a1, a2);
+                };
+                const double d1 = exact(m), d2 = exact(q2), d3 = exact(up(q2)), d4 = exact(up(m));
+                f = edge_theta(d1, d2) + edge_theta(d2, d3) + edge_theta(d3, d4) > accept;
+            }
+        }
+        const uint64_t w = __ballot(f);
+        const uint32_t wi = (base + 64u * t) / 64;
+        if (lane == 0 && (uint64_t)wi * 64 < L) words[wi] = w;
+        total += (uint32_t)__popcll(w);
+    }
+    if (!bcount) return;                                     // uniform over the grid
+    if (lane == 0) wave_tot[wave] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int w = 0; w < kStrBlock / 64; ++w) t += wave_tot[w];
+        bcount[blk] = t;
+    }
+}
+
+template <class P>
+__global__ void __launch_bounds__(kStrBlock)
+strings2d_kernel(int N, uint32_t L, P phi, double accept, uint64_t *__restrict__ words,
+                 uint32_t *__restrict__ bcount)
+{
+    strings2d_block(N, L, phi, accept, words, bcount, blockIdx.x);
+}
+
+template <class P>
+__global__ void __launch_bounds__(kStrBlock)
+strings2d_batch_kernel(const StrMember *__restrict__ mem, const uint32_t *__restrict__ blk2mem,
+                       int half, double accept, uint64_t *__restrict__ words)
+{
+    const StrMember *M = mem + blk2mem[blockIdx.x];
+    P phi;
+    phi.p = (decltype(phi.p))M->phi[half];
+    strings2d_block(M->N, M->L, phi, accept, words + (size_t)M->first_block * (kStrSpan / 64),
+                    (uint32_t *)nullptr, blockIdx.x - M->first_block);
 }
 
 template <class P, bool ALIGNED>
@@ -432,7 +421,9 @@ block_counts_kernel(const uint64_t *__restrict__ words, uint64_t nwords, uint32_
 // per work-item) to tile-relative offsets and tile sums; top_scan_kernel
 // scans the tile sums (one per work-item: lattices hold fewer than 2^31
 // sites, so n <= 2^20 and there are at most 256 tiles) and writes the
-// total; add_tile_offsets_kernel adds each tile's offset.
+// total; add_tile_offsets_kernel adds each tile's offset.  One tile (up to
+// 8M sites) takes the first launch alone.  The total also goes to the
+// context's pinned mailbox (*total), so no copy follows.
 constexpr int kScanTile = 4096;
 
 // exclusive prefix of v over the 1024 work-items; *total gets the sum
@@ -464,7 +455,7 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T *lds, T *total)
 
 __global__ void __launch_bounds__(1024)
 tile_scan_kernel(const uint32_t *__restrict__ cnt, uint64_t *__restrict__ off,
-                 uint64_t *__restrict__ tsum, uint32_t n)
+                 uint64_t *__restrict__ tsum, uint32_t n, uint64_t *__restrict__ total)
 {
     __shared__ uint32_t lds[17];
     const uint32_t e0 = blockIdx.x * (uint32_t)kScanTile + 4u * threadIdx.x;
@@ -479,18 +470,28 @@ tile_scan_kernel(const uint32_t *__restrict__ cnt, uint64_t *__restrict__ off,
         if (e0 + u < n) off[e0 + u] = acc;
         acc += c[u];
     }
-    if (threadIdx.x == 0) tsum[blockIdx.x] = tot;
+    if (threadIdx.x == 0) {
+        tsum[blockIdx.x] = tot;
+        if (total) {                     // a single tile: the scan is complete
+            off[n] = tot;
+            *total = tot;
+        }
+    }
 }
 
 __global__ void __launch_bounds__(1024)
-top_scan_kernel(uint64_t *__restrict__ tsum, uint32_t ntiles, uint64_t *__restrict__ total)
+top_scan_kernel(uint64_t *__restrict__ tsum, uint32_t ntiles, uint64_t *__restrict__ last,
+                uint64_t *__restrict__ total)
 {
     __shared__ uint64_t lds[17];
     const uint64_t v = (threadIdx.x < ntiles) ? tsum[threadIdx.x] : 0ull;
     uint64_t tot;
     const uint64_t x = block_exclusive_scan<uint64_t>(v, lds, &tot);
     if (threadIdx.x < ntiles) tsum[threadIdx.x] = x;
-    if (threadIdx.x == 0) *total = tot;
+    if (threadIdx.x == 0) {
+        *last = tot;
+        *total = tot;
+    }
 }
 
 __global__ void __launch_bounds__(256)
@@ -588,17 +589,21 @@ __device__ __forceinline__ void count_word(const uint64_t *__restrict__ words, u
     }
 }
 
-template <int ND>
-__global__ void __launch_bounds__(256)
+// one work-group over a small lattice's words (kCountAlone at most): the
+// counts go straight to cnt, with nothing to clear before or copy after
+constexpr uint64_t kCountAlone = 16384;
+
+template <int ND, int BLOCK, bool ALONE>
+__global__ void __launch_bounds__(BLOCK)
 member_count_kernel(const uint64_t *__restrict__ words, uint32_t L, int N,
                     unsigned long long *__restrict__ cnt)
 {
-    __shared__ unsigned long long part[2][4];
+    __shared__ unsigned long long part[2][BLOCK / 64];
     const uint64_t nwords = ((uint64_t)L + 63) / 64;
     unsigned long long n = 0, pairs = 0;
     // grid-stride over the words, one pair of atomics per work-group
-    for (uint64_t w = blockIdx.x * 256ull + threadIdx.x; w < nwords;
-         w += (uint64_t)gridDim.x * 256ull)
+    for (uint64_t w = blockIdx.x * (uint64_t)BLOCK + threadIdx.x; w < nwords;
+         w += (uint64_t)gridDim.x * (uint64_t)BLOCK)
         count_word<ND>(words, nwords, N, w, n, pairs);
     for (int o = 32; o > 0; o >>= 1) {
         n += __shfl_down(n, o, 64);
@@ -611,10 +616,18 @@ member_count_kernel(const uint64_t *__restrict__ words, uint32_t L, int N,
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        const unsigned long long tn = part[0][0] + part[0][1] + part[0][2] + part[0][3];
-        const unsigned long long tp = part[1][0] + part[1][1] + part[1][2] + part[1][3];
-        if (tn) atomicAdd(&cnt[0], tn);
-        if (tp) atomicAdd(&cnt[1], tp);
+        unsigned long long tn = 0, tp = 0;
+        for (int w = 0; w < BLOCK / 64; ++w) {
+            tn += part[0][w];
+            tp += part[1][w];
+        }
+        if (ALONE) {
+            cnt[0] = tn;
+            cnt[1] = tp;
+        } else {
+            if (tn) atomicAdd(&cnt[0], tn);
+            if (tp) atomicAdd(&cnt[1], tp);
+        }
     }
 }
 
@@ -653,20 +666,19 @@ static double accept_threshold(int thr)
     return (double)f;
 }
 
-// one-pass 3D finder: ballot words of every site, then the per-block
-// counts the scan and the coordinate writer use
+// one-pass 3D finder: ballot words of every site
 static int launch_strings_march(Context *c, int N, uint32_t L, const void *phi, double accept,
-                                uint64_t *words, uint32_t *bcount)
+                                uint64_t *words)
 {
     SfGeom g;
     g.N = N;
     g.nTj = (N + kSfTJ - 1) / kSfTJ;
     g.nTk = (N + 63) / 64;
     const uint64_t tiles = (uint64_t)g.nTj * (uint64_t)g.nTk;
-    // longest chunk (64 planes down to 4) that still gives two work-groups
+    // longest chunk (64 planes down to 1) that still gives two work-groups
     // per CU: the first plane of each chunk is the previous chunk's last
     int CI = 64;
-    while (CI > 4 && tiles * (uint64_t)((N + CI - 1) / CI) < 2 * (uint64_t)c->num_cu) CI >>= 1;
+    while (CI > 1 && tiles * (uint64_t)((N + CI - 1) / CI) < 2 * (uint64_t)c->num_cu) CI >>= 1;
     g.CI = CI;
     const uint32_t grid = (uint32_t)(tiles * (uint64_t)((N + CI - 1) / CI));
     const uint64_t nwords = ((uint64_t)L + 63) / 64;
@@ -687,8 +699,6 @@ static int launch_strings_march(Context *c, int N, uint32_t L, const void *phi, 
             hipLaunchKernelGGL((strings_march_kernel<PhiF32, false>), dim3(grid), dim3(64 * kSfW),
                                0, c->stream, g, PhiF32{(const fvec4 *)phi}, accept, w);
     }
-    hipLaunchKernelGGL(block_counts_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0,
-                       c->stream, words, nwords, bcount);
     AXS_HIP_TRY(hipGetLastError());
     return AXS_OK;
 }
@@ -714,7 +724,8 @@ struct StrLayout {
     size_t bytes() const { return words_b + cnt_b + off_b + tail_b + counters_b; }
 };
 
-// ballot words and block counts of member m (the search itself)
+// ballot words of member m (the search itself); 2D also the block counts
+// that a coordinate list's scan needs (3D: block_counts_kernel before the scan)
 static int search_member(Context *c, Member &m, uint64_t *words, uint32_t *bcount)
 {
     const uint32_t L = (uint32_t)m.L;
@@ -722,21 +733,13 @@ static int search_member(Context *c, Member &m, uint64_t *words, uint32_t *bcoun
     // the angles need phi only (no FP32 velocity reconstruction)
     const void *phi = m.state[c->cur][PHI];
     const double accept = accept_threshold(c->p.thr);
-    if (c->nd == 3) return launch_strings_march(c, m.N, L, phi, accept, words, bcount);
-    AXS_TRY(ensure_scratch(c, (size_t)L * sizeof(double)));
-    double *ang = (double *)c->scratch;
-    const unsigned ga = (L + 255) / 256;
-    if (c->prec == AXS_FP64) {
-        const PhiF64 p{(const dvec2 *)phi};
-        hipLaunchKernelGGL(angle_kernel<PhiF64>, dim3(ga), dim3(256), 0, c->stream, L, p, ang);
-        hipLaunchKernelGGL(strings_flag_kernel<PhiF64>, dim3(nblocks), dim3(kStrBlock), 0,
-                           c->stream, m.N, L, ang, p, accept, words, bcount);
-    } else {
-        const PhiF32 p{(const fvec4 *)phi};
-        hipLaunchKernelGGL(angle_kernel<PhiF32>, dim3(ga), dim3(256), 0, c->stream, L, p, ang);
-        hipLaunchKernelGGL(strings_flag_kernel<PhiF32>, dim3(nblocks), dim3(kStrBlock), 0,
-                           c->stream, m.N, L, ang, p, accept, words, bcount);
-    }
+    if (c->nd == 3) return launch_strings_march(c, m.N, L, phi, accept, words);
+    if (c->prec == AXS_FP64)
+        hipLaunchKernelGGL(strings2d_kernel<PhiF64>, dim3(nblocks), dim3(kStrBlock), 0, c->stream,
+                           m.N, L, PhiF64{(const dvec2 *)phi}, accept, words, bcount);
+    else
+        hipLaunchKernelGGL(strings2d_kernel<PhiF32>, dim3(nblocks), dim3(kStrBlock), 0, c->stream,
+                           m.N, L, PhiF32{(const fvec4 *)phi}, accept, words, bcount);
     AXS_HIP_TRY(hipGetLastError());
     return AXS_OK;
 }
@@ -762,6 +765,8 @@ int run_axion(Context *c, Member &m, double *out)
     return copy_to_host(c, out, d, (size_t)L * sizeof(double));
 }
 
+constexpr size_t kListDirect = (size_t)256 << 10;
+
 int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *count,
                 int64_t *num_cores)
 {
@@ -786,11 +791,17 @@ int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *co
     unsigned long long *pairs = (unsigned long long *)(sp + lay.words_b + lay.cnt_b + lay.off_b);
     uint64_t *tsum = (uint64_t *)(sp + lay.words_b + lay.cnt_b + lay.off_b + 256);
 
+    uint64_t *mail = (uint64_t *)c->mail;
     auto scan = [&]() {
+        const uint64_t nwords = ((uint64_t)L + 63) / 64;
+        if (c->nd == 3)
+            hipLaunchKernelGGL(block_counts_kernel, dim3((unsigned)((nwords + 255) / 256)),
+                               dim3(256), 0, c->stream, words, nwords, bcount);
         hipLaunchKernelGGL(tile_scan_kernel, dim3(ntiles), dim3(1024), 0, c->stream, bcount, off,
-                           tsum, nblocks);
+                           tsum, nblocks, (ntiles == 1) ? mail : (uint64_t *)nullptr);
+        if (ntiles == 1) return hipGetLastError();
         hipLaunchKernelGGL(top_scan_kernel, dim3(1), dim3(1024), 0, c->stream, tsum, ntiles,
-                           off + nblocks);
+                           off + nblocks, mail);
         hipLaunchKernelGGL(add_tile_offsets_kernel, dim3((nblocks + 255) / 256), dim3(256), 0,
                            c->stream, off, tsum, nblocks);
         return hipGetLastError();
@@ -801,8 +812,8 @@ int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *co
     } else {
         AXS_TRY(search_member(c, m, words, bcount));
         AXS_HIP_TRY(scan());
-        AXS_HIP_TRY(hipMemcpyAsync(&total, off + nblocks, 8, hipMemcpyDeviceToHost, c->stream));
         AXS_HIP_TRY(hipStreamSynchronize(c->stream));
+        total = *(volatile uint64_t *)mail;
         c->str_member = member;
         c->str_version = m.version;
         c->str_total = total;
@@ -820,10 +831,16 @@ int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *co
         c->str_scanned = true;
     }
 
-    // coordinate list in its own buffer (scratch keeps words / offsets)
-    size_t list_b = (size_t)total * c->nd * sizeof(int32_t) + 256;
-    AXS_TRY(ensure_device(c, &c->listbuf, &c->listbuf_bytes, list_b));
-    int32_t *dlist = (int32_t *)c->listbuf;
+    // coordinate list in its own buffer (scratch keeps words / offsets); a
+    // small one that only goes to the host is written to pinned memory
+    // directly, which saves a copy's launch and wait (256^2: 8 us)
+    const size_t list_b = (size_t)total * c->nd * sizeof(int32_t) + 256;
+    const bool direct = list_b <= kListDirect && num_cores == nullptr;
+    if (direct)
+        AXS_TRY(ensure_pinned(c, kListDirect));
+    else
+        AXS_TRY(ensure_device(c, &c->listbuf, &c->listbuf_bytes, list_b));
+    int32_t *dlist = (int32_t *)(direct ? c->pinned : c->listbuf);
 
     if (total > 0) {
         auto kw = (c->nd == 2) ? strings_write_kernel<2> : strings_write_kernel<3>;
@@ -850,29 +867,28 @@ int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *co
 
     if (coords && cap > 0) {
         int64_t ncopy = (cap < (int64_t)total) ? cap : (int64_t)total;
-        if (ncopy > 0)
+        if (ncopy > 0 && !direct)
             AXS_TRY(copy_to_host(c, coords, dlist, (size_t)ncopy * c->nd * sizeof(int32_t)));
         AXS_HIP_TRY(hipStreamSynchronize(c->stream));
+        if (ncopy > 0 && direct)
+            memcpy(coords, dlist, (size_t)ncopy * c->nd * sizeof(int32_t));
     }
     return (coords == nullptr || cap >= (int64_t)total) ? AXS_OK : AXS_ERR_CAPACITY;
 }
 
-// axs_string_counts of a 2D ensemble: three launches for all members (the
-// angles, the plaquette test and the counts over the concatenated block
-// space), one copy, one synchronisation
+// axs_string_counts of a 2D ensemble: two launches for all members (the
+// plaquette test and the counts over the concatenated block space), one copy,
+// one synchronisation
 static int run_string_counts_2d_batch(Context *c, int64_t *n_plaquettes, int64_t *num_cores)
 {
     const size_t nm = c->members.size();
     auto align = [](size_t x) { return (x + 255) & ~(size_t)255; };
     std::vector<StrMember> tab(nm);
     uint32_t nblocks = 0;
-    uint64_t sites = 0;
     for (size_t r = 0; r < nm; ++r) {
         const Member &m = c->members[r];
-        tab[r] = StrMember{{m.state[0][PHI], m.state[1][PHI]}, sites, (uint32_t)m.L, nblocks,
-                           m.N, 0};
+        tab[r] = StrMember{{m.state[0][PHI], m.state[1][PHI]}, (uint32_t)m.L, nblocks, m.N, 0};
         nblocks += ((uint32_t)m.L + kStrSpan - 1) / kStrSpan;
-        sites += (uint64_t)m.L;
     }
     const size_t tab_b = align(nm * sizeof(StrMember));
     if (!c->strtab) {          // members and their buffers are fixed: built once
@@ -890,33 +906,25 @@ static int run_string_counts_2d_batch(Context *c, int64_t *n_plaquettes, int64_t
     }
     const StrMember *dmem = (const StrMember *)c->strtab;
     const uint32_t *dblk = (const uint32_t *)((char *)c->strtab + tab_b);
-    const size_t words_b = (size_t)nblocks * (kStrSpan / 64) * 8, cnt_b = align((size_t)nblocks * 4);
+    const size_t words_b = (size_t)nblocks * (kStrSpan / 64) * 8;
     c->str_member = -1;
-    AXS_TRY(ensure_device(c, &c->strbuf, &c->strbuf_bytes, words_b + cnt_b + align(nm * 16)));
-    AXS_TRY(ensure_scratch(c, (size_t)sites * sizeof(double)));
+    AXS_TRY(ensure_device(c, &c->strbuf, &c->strbuf_bytes, words_b + align(nm * 16)));
     char *sp = (char *)c->strbuf;
     uint64_t *words = (uint64_t *)sp;
-    uint32_t *bcount = (uint32_t *)(sp + words_b);
-    unsigned long long *counters = (unsigned long long *)(sp + words_b + cnt_b);
-    double *ang = (double *)c->scratch;
+    unsigned long long *counters = (unsigned long long *)(sp + words_b);
     AXS_HIP_TRY(hipMemsetAsync(counters, 0, nm * 16, c->stream));
     const double accept = accept_threshold(c->p.thr);
-    if (c->prec == AXS_FP64) {
-        hipLaunchKernelGGL(angle_batch_kernel<PhiF64>, dim3(nblocks), dim3(kStrBlock), 0,
-                           c->stream, dmem, dblk, c->cur, ang);
-        hipLaunchKernelGGL(strings_flag_batch_kernel<PhiF64>, dim3(nblocks), dim3(kStrBlock), 0,
-                           c->stream, dmem, dblk, c->cur, ang, accept, words, bcount);
-    } else {
-        hipLaunchKernelGGL(angle_batch_kernel<PhiF32>, dim3(nblocks), dim3(kStrBlock), 0,
-                           c->stream, dmem, dblk, c->cur, ang);
-        hipLaunchKernelGGL(strings_flag_batch_kernel<PhiF32>, dim3(nblocks), dim3(kStrBlock), 0,
-                           c->stream, dmem, dblk, c->cur, ang, accept, words, bcount);
-    }
+    if (c->prec == AXS_FP64)
+        hipLaunchKernelGGL(strings2d_batch_kernel<PhiF64>, dim3(nblocks), dim3(kStrBlock), 0,
+                           c->stream, dmem, dblk, c->cur, accept, words);
+    else
+        hipLaunchKernelGGL(strings2d_batch_kernel<PhiF32>, dim3(nblocks), dim3(kStrBlock), 0,
+                           c->stream, dmem, dblk, c->cur, accept, words);
     hipLaunchKernelGGL(count_batch_kernel, dim3((nblocks + 7) / 8), dim3(256), 0, c->stream, dmem,
                        dblk, nblocks, words, counters);
     AXS_HIP_TRY(hipGetLastError());
-    std::vector<unsigned long long> h(2 * nm);
-    AXS_HIP_TRY(hipMemcpyAsync(h.data(), counters, nm * 16, hipMemcpyDeviceToHost, c->stream));
+    unsigned long long *h = (unsigned long long *)c->mail;
+    AXS_HIP_TRY(hipMemcpyAsync(h, counters, nm * 16, hipMemcpyDeviceToHost, c->stream));
     AXS_HIP_TRY(hipStreamSynchronize(c->stream));
     for (size_t r = 0; r < nm; ++r) {
         if (n_plaquettes) n_plaquettes[r] = (int64_t)h[2 * r];
@@ -944,12 +952,16 @@ int run_string_counts(Context *c, int64_t *n_plaquettes, int64_t *num_cores)
     const StrLayout lay(Lmax, nm);
     c->str_member = -1;
     AXS_TRY(ensure_device(c, &c->strbuf, &c->strbuf_bytes, lay.bytes()));
-    if (c->nd == 2) AXS_TRY(ensure_scratch(c, (size_t)Lmax * sizeof(double)));
     char *sp = (char *)c->strbuf;
     uint64_t *words = (uint64_t *)sp;
+    // counters in the pinned mailbox where every member's words fit one
+    // work-group (nothing to clear, no copy), else on the device
+    const bool alone = ((uint64_t)Lmax + 63) / 64 <= kCountAlone;
+    unsigned long long *h = (unsigned long long *)c->mail;
     unsigned long long *counters =
-        (unsigned long long *)(sp + lay.words_b + lay.cnt_b + lay.off_b + lay.tail_b);
-    AXS_HIP_TRY(hipMemsetAsync(counters, 0, nm * 16, c->stream));
+        alone ? h
+              : (unsigned long long *)(sp + lay.words_b + lay.cnt_b + lay.off_b + lay.tail_b);
+    if (!alone) AXS_HIP_TRY(hipMemsetAsync(counters, 0, nm * 16, c->stream));
     for (size_t r = 0; r < nm; ++r) {
         Member &m = c->members[r];
         // block counts where the member's own layout keeps them (below the
@@ -959,13 +971,22 @@ int run_string_counts(Context *c, int64_t *n_plaquettes, int64_t *num_cores)
         AXS_TRY(search_member(c, m, words, (uint32_t *)(sp + lr.words_b)));
         const uint32_t L = (uint32_t)m.L;
         const uint64_t nw = ((uint64_t)L + 63) / 64;
-        const unsigned g = (unsigned)std::min<uint64_t>((nw + 255) / 256, 4ull * c->num_cu);
-        auto k = (c->nd == 2) ? member_count_kernel<2> : member_count_kernel<3>;
-        hipLaunchKernelGGL(k, dim3(g), dim3(256), 0, c->stream, words, L, m.N, counters + 2 * r);
+        if (alone) {
+            auto k = (c->nd == 2) ? member_count_kernel<2, 1024, true>
+                                  : member_count_kernel<3, 1024, true>;
+            hipLaunchKernelGGL(k, dim3(1), dim3(1024), 0, c->stream, words, L, m.N,
+                               counters + 2 * r);
+        } else {
+            const unsigned g = (unsigned)std::min<uint64_t>((nw + 255) / 256, 4ull * c->num_cu);
+            auto k = (c->nd == 2) ? member_count_kernel<2, 256, false>
+                                  : member_count_kernel<3, 256, false>;
+            hipLaunchKernelGGL(k, dim3(g), dim3(256), 0, c->stream, words, L, m.N,
+                               counters + 2 * r);
+        }
         AXS_HIP_TRY(hipGetLastError());
     }
-    std::vector<unsigned long long> h(2 * nm);
-    AXS_HIP_TRY(hipMemcpyAsync(h.data(), counters, nm * 16, hipMemcpyDeviceToHost, c->stream));
+    if (!alone)
+        AXS_HIP_TRY(hipMemcpyAsync(h, counters, nm * 16, hipMemcpyDeviceToHost, c->stream));
     AXS_HIP_TRY(hipStreamSynchronize(c->stream));
     for (size_t r = 0; r < nm; ++r) {
         if (n_plaquettes) n_plaquettes[r] = (int64_t)h[2 * r];
