@@ -135,147 +135,96 @@ int ensure_pinned(Context *c, size_t bytes)
     return AXS_OK;
 }
 
-struct HostCopy {
-    char *dst;
-    const char *src;
+// host-side (de)interleaving between the reference's separate double arrays
+// and the staged device layouts, sites [lo, lo + n)
+
+// FP64 pairs; either source may be null (zero), either destination (skip)
+struct Pair64 {
+    const double *a, *b;
+    double *oa, *ob;
 };
 
-static void host_copy_fn(size_t lo, size_t hi, void *arg)
+static void pack64_fn(char *stage, size_t lo, size_t n, void *arg)
 {
-    HostCopy *h = (HostCopy *)arg;
-    memcpy(h->dst + lo, h->src + lo, hi - lo);
-}
-
-int copy_to_host(Context *c, void *dst, const void *src, size_t bytes)
-{
-    constexpr size_t kChunk = (size_t)64 << 20;
-    if (bytes <= kChunk) {
-        AXS_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-        AXS_HIP_TRY(hipStreamSynchronize(c->stream));
-        return AXS_OK;
-    }
-    AXS_TRY(ensure_pinned(c, 2 * kChunk));
-    for (int h = 0; h < 2; ++h)
-        if (!c->stage_ev[h]) AXS_HIP_TRY(hipEventCreateWithFlags(&c->stage_ev[h],
-                                                                 hipEventDisableTiming));
-    char *stage[2] = {(char *)c->pinned, (char *)c->pinned + kChunk};
-    const size_t n = (bytes + kChunk - 1) / kChunk;
-    auto chunk_bytes = [&](size_t q) { return std::min(kChunk, bytes - q * kChunk); };
-    // chunk q goes to stage q % 2; it is copied out after chunk q+1 is queued
-    AXS_HIP_TRY(hipMemcpyAsync(stage[0], src, chunk_bytes(0), hipMemcpyDeviceToHost, c->stream));
-    AXS_HIP_TRY(hipEventRecord(c->stage_ev[0], c->stream));
-    for (size_t q = 0; q < n; ++q) {
-        const int h = (int)(q & 1);
-        if (q + 1 < n) {
-            const size_t nb = chunk_bytes(q + 1);
-            AXS_HIP_TRY(hipMemcpyAsync(stage[h ^ 1], (const char *)src + (q + 1) * kChunk, nb,
-                                       hipMemcpyDeviceToHost, c->stream));
-            AXS_HIP_TRY(hipEventRecord(c->stage_ev[h ^ 1], c->stream));
+    const Pair64 *p = (const Pair64 *)arg;
+    double *__restrict__ d = (double *)stage;
+    const double *__restrict__ a = p->a ? p->a + lo : nullptr;
+    const double *__restrict__ b = p->b ? p->b + lo : nullptr;
+    if (a && b) {
+        for (size_t i = 0; i < n; ++i) {
+            d[2 * i] = a[i];
+            d[2 * i + 1] = b[i];
         }
-        AXS_HIP_TRY(hipEventSynchronize(c->stage_ev[h]));
-        HostCopy hc{(char *)dst + q * kChunk, stage[h]};
-        parallel_for(chunk_bytes(q), host_copy_fn, &hc);
-        // stage h is free again only after its copy-out: the transfer of
-        // chunk q+2 into it is queued in the next iteration, after this one
-    }
-    return AXS_OK;
-}
-
-void parallel_for(size_t n, void (*fn)(size_t, size_t, void *), void *arg)
-{
-    unsigned hw = std::thread::hardware_concurrency();
-    unsigned nt = hw ? std::min(hw, 16u) : 4u;
-    if (n < ((size_t)1 << 20) || nt <= 1) {
-        fn(0, n, arg);
         return;
     }
-    std::vector<std::thread> ts;
-    size_t chunk = (n + nt - 1) / nt;
-    for (unsigned t = 0; t < nt; ++t) {
-        size_t b = t * chunk, e = std::min(n, b + chunk);
-        if (b >= e) break;
-        ts.emplace_back(fn, b, e, arg);
-    }
-    for (auto &t : ts) t.join();
-}
-
-// host-side (de)interleaving between the reference's separate double
-// arrays and the device layouts
-struct Pack64 {
-    double *dst;              // pairs
-    const double *a, *b;      // either may be null (zero)
-};
-
-static void pack64_fn(size_t lo, size_t hi, void *arg)
-{
-    Pack64 *c = (Pack64 *)arg;
-    for (size_t i = lo; i < hi; ++i) {
-        c->dst[2 * i] = c->a ? c->a[i] : 0.0;
-        c->dst[2 * i + 1] = c->b ? c->b[i] : 0.0;
+    for (size_t i = 0; i < n; ++i) {
+        d[2 * i] = a ? a[i] : 0.0;
+        d[2 * i + 1] = b ? b[i] : 0.0;
     }
 }
 
-struct Unpack64 {
-    const double *src;        // pairs
-    double *a, *b;            // either may be null (skip)
-};
-
-static void unpack64_fn(size_t lo, size_t hi, void *arg)
+static void unpack64_fn(char *stage, size_t lo, size_t n, void *arg)
 {
-    Unpack64 *c = (Unpack64 *)arg;
-    for (size_t i = lo; i < hi; ++i) {
-        if (c->a) c->a[i] = c->src[2 * i];
-        if (c->b) c->b[i] = c->src[2 * i + 1];
+    const Pair64 *p = (const Pair64 *)arg;
+    const double *__restrict__ s = (const double *)stage;
+    double *__restrict__ a = p->oa ? p->oa + lo : nullptr;
+    double *__restrict__ b = p->ob ? p->ob + lo : nullptr;
+    if (a && b) {
+        for (size_t i = 0; i < n; ++i) {
+            a[i] = s[2 * i];
+            b[i] = s[2 * i + 1];
+        }
+        return;
+    }
+    for (size_t i = 0; i < n; ++i) {
+        if (a) a[i] = s[2 * i];
+        if (b) b[i] = s[2 * i + 1];
     }
 }
 
 // FP32 state quadruple (phi1, phi2, u1, u2), u = phidot + dt/2 ker (in double)
 struct Pack32 {
-    float *dst;
     const double *p1, *p2, *v1, *v2, *k1, *k2;
     double half_dt;
 };
 
-static void pack32_fn(size_t lo, size_t hi, void *arg)
+static void pack32_fn(char *stage, size_t lo, size_t n, void *arg)
 {
-    Pack32 *c = (Pack32 *)arg;
-    for (size_t i = lo; i < hi; ++i) {
-        double u1 = c->v1[i], u2 = c->v2[i];
-        if (c->k1) u1 = u1 + c->half_dt * c->k1[i];
-        if (c->k2) u2 = u2 + c->half_dt * c->k2[i];
-        c->dst[4 * i] = (float)c->p1[i];
-        c->dst[4 * i + 1] = (float)c->p2[i];
-        c->dst[4 * i + 2] = (float)u1;
-        c->dst[4 * i + 3] = (float)u2;
+    const Pack32 *c = (const Pack32 *)arg;
+    float *__restrict__ d = (float *)stage;
+    for (size_t i = 0; i < n; ++i) {
+        const size_t m = lo + i;
+        double u1 = c->v1[m], u2 = c->v2[m];
+        if (c->k1) u1 = u1 + c->half_dt * c->k1[m];
+        if (c->k2) u2 = u2 + c->half_dt * c->k2[m];
+        d[4 * i] = (float)c->p1[m];
+        d[4 * i + 1] = (float)c->p2[m];
+        d[4 * i + 2] = (float)u1;
+        d[4 * i + 3] = (float)u2;
     }
 }
 
-struct PackPair32 {
-    float *dst;
-    const double *a, *b;
-};
-
-static void packpair32_fn(size_t lo, size_t hi, void *arg)
+static void packpair32_fn(char *stage, size_t lo, size_t n, void *arg)
 {
-    PackPair32 *c = (PackPair32 *)arg;
-    for (size_t i = lo; i < hi; ++i) {
-        c->dst[2 * i] = c->a ? (float)c->a[i] : 0.0f;
-        c->dst[2 * i + 1] = c->b ? (float)c->b[i] : 0.0f;
+    const Pair64 *p = (const Pair64 *)arg;
+    float *__restrict__ d = (float *)stage;
+    for (size_t i = 0; i < n; ++i) {
+        d[2 * i] = p->a ? (float)p->a[lo + i] : 0.0f;
+        d[2 * i + 1] = p->b ? (float)p->b[lo + i] : 0.0f;
     }
 }
 
-struct Unpack32 {
-    const float *src;
-    int stride;               // 4 for the state, 2 for pairs
-    double *a, *b;
-};
-
-static void unpack32_fn(size_t lo, size_t hi, void *arg)
+// the first pair of every STRIDE floats, widened
+template <int STRIDE>
+static void unpack32_fn(char *stage, size_t lo, size_t n, void *arg)
 {
-    Unpack32 *c = (Unpack32 *)arg;
-    for (size_t i = lo; i < hi; ++i) {
-        if (c->a) c->a[i] = (double)c->src[c->stride * i];
-        if (c->b) c->b[i] = (double)c->src[c->stride * i + 1];
+    const Pair64 *p = (const Pair64 *)arg;
+    const float *__restrict__ s = (const float *)stage;
+    double *__restrict__ a = p->oa ? p->oa + lo : nullptr;
+    double *__restrict__ b = p->ob ? p->ob + lo : nullptr;
+    for (size_t i = 0; i < n; ++i) {
+        if (a) a[i] = (double)s[STRIDE * i];
+        if (b) b[i] = (double)s[STRIDE * i + 1];
     }
 }
 
@@ -286,6 +235,7 @@ Context::~Context()
 {
     if (stream) (void)hipStreamSynchronize(stream);
     destroy_snapshot(this);
+    destroy_pool(this);
     destroy_plans(this);
     destroy_inverse_plans(this);
     destroy_spec_plans(this);
@@ -315,8 +265,8 @@ Context::~Context()
     if (mail) (void)hipHostFree(mail);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
-    for (int h = 0; h < 2; ++h)
-        if (stage_ev[h]) (void)hipEventDestroy(stage_ev[h]);
+    for (hipEvent_t e : stage_ev)
+        if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -629,27 +579,23 @@ int axs_set_member_state(axs_ctx *ctx, int member, const double *phi1, const dou
     }
     Context *c = &ctx->impl;
     Member &m = c->members[member];
-    size_t L = (size_t)m.L;
-    int h = c->cur;
-    AXS_TRY(ensure_pinned(c, L * 16));
+    const size_t L = (size_t)m.L;
+    const int h = c->cur;
     if (c->prec == AXS_FP64) {
-        double *st = (double *)c->pinned;
-        const double *srcs[3][2] = {{phi1, phi2}, {phidot1, phidot2}, {ker1, ker2}};
-        for (int a = 0; a < 3; ++a) {
-            Pack64 pk{st, srcs[a][0], srcs[a][1]};
-            parallel_for(L, pack64_fn, &pk);
-            AXS_HIP_TRY(hipMemcpy(m.state[h][a], st, L * 16, hipMemcpyHostToDevice));
-        }
+        Pair64 pr[3] = {{phi1, phi2, nullptr, nullptr},
+                        {phidot1, phidot2, nullptr, nullptr},
+                        {ker1, ker2, nullptr, nullptr}};
+        Segment sg[3];
+        for (int a = 0; a < 3; ++a) sg[a] = Segment{m.state[h][a], 16, L, pack64_fn, &pr[a]};
+        AXS_TRY(transfer(c, sg, 3, false));
     } else {
         // FP32 form: u = phidot + dt/2 ker in double, rounded once; ker kept
         // for the state read-back before the first step
-        float *st = (float *)c->pinned;
-        Pack32 pk{st, phi1, phi2, phidot1, phidot2, ker1, ker2, 0.5 * (double)c->p.time_step};
-        parallel_for(L, pack32_fn, &pk);
-        AXS_HIP_TRY(hipMemcpy(m.state[h][PHI], st, L * 16, hipMemcpyHostToDevice));
-        PackPair32 kp{st, ker1, ker2};
-        parallel_for(L, packpair32_fn, &kp);
-        AXS_HIP_TRY(hipMemcpy(m.aux_ker, st, L * 8, hipMemcpyHostToDevice));
+        Pack32 pk{phi1, phi2, phidot1, phidot2, ker1, ker2, 0.5 * (double)c->p.time_step};
+        Pair64 kp{ker1, ker2, nullptr, nullptr};
+        const Segment sg[2] = {Segment{m.state[h][PHI], 16, L, pack32_fn, &pk},
+                               Segment{m.aux_ker, 8, L, packpair32_fn, &kp}};
+        AXS_TRY(transfer(c, sg, 2, false));
         m.ker_valid = true;
         m.ker_uploaded = true;
     }
@@ -669,41 +615,25 @@ int axs_get_member_state(axs_ctx *ctx, int member, double *phi1, double *phi2, d
         set_error("member %d has no state", member);
         return AXS_ERR_STATE;
     }
-    size_t L = (size_t)m.L;
-    int h = c->cur;
-    AXS_TRY(ensure_pinned(c, L * 16));
+    const size_t L = (size_t)m.L;
+    const int h = c->cur;
+    Pair64 pr[3] = {{nullptr, nullptr, phi1, phi2},
+                    {nullptr, nullptr, phidot1, phidot2},
+                    {nullptr, nullptr, ker1, ker2}};
+    Segment all[3], want[3];
     if (c->prec == AXS_FP64) {
-        double *st = (double *)c->pinned;
-        double *dst[3][2] = {{phi1, phi2}, {phidot1, phidot2}, {ker1, ker2}};
-        for (int a = 0; a < 3; ++a) {
-            if (!dst[a][0] && !dst[a][1]) continue;
-            AXS_HIP_TRY(hipMemcpyAsync(st, m.state[h][a], L * 16, hipMemcpyDeviceToHost,
-                                       c->stream));
-            AXS_HIP_TRY(hipStreamSynchronize(c->stream));
-            Unpack64 up{st, dst[a][0], dst[a][1]};
-            parallel_for(L, unpack64_fn, &up);
-        }
-        return AXS_OK;
+        for (int a = 0; a < 3; ++a) all[a] = Segment{m.state[h][a], 16, L, unpack64_fn, &pr[a]};
+    } else {
+        FieldView fv;
+        AXS_TRY(current_fields(c, m, &fv));      // rebuilds ker and phidot
+        all[0] = Segment{m.state[h][PHI], 16, L, unpack32_fn<4>, &pr[0]};
+        all[1] = Segment{m.aux_vel, 8, L, unpack32_fn<2>, &pr[1]};
+        all[2] = Segment{m.aux_ker, 8, L, unpack32_fn<2>, &pr[2]};
     }
-    FieldView fv;
-    AXS_TRY(current_fields(c, m, &fv));      // rebuilds ker and phidot
-    float *st = (float *)c->pinned;
-    struct {
-        const void *src;
-        size_t bytes;
-        int stride;
-        double *a, *b;
-    } jobs[3] = {{m.state[h][PHI], L * 16, 4, phi1, phi2},
-                 {m.aux_vel, L * 8, 2, phidot1, phidot2},
-                 {m.aux_ker, L * 8, 2, ker1, ker2}};
-    for (auto &j : jobs) {
-        if (!j.a && !j.b) continue;
-        AXS_HIP_TRY(hipMemcpyAsync(st, j.src, j.bytes, hipMemcpyDeviceToHost, c->stream));
-        AXS_HIP_TRY(hipStreamSynchronize(c->stream));
-        Unpack32 up{st, j.stride, j.a, j.b};
-        parallel_for(L, unpack32_fn, &up);
-    }
-    return AXS_OK;
+    int n = 0;
+    for (int a = 0; a < 3; ++a)
+        if (pr[a].oa || pr[a].ob) want[n++] = all[a];
+    return transfer(c, want, n, true);
 }
 
 int axs_init_member(axs_ctx *ctx, int member, int mode, uint64_t seed)

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -113,6 +114,7 @@ struct Member {
 };
 
 struct FftPlan;
+struct HostPool;
 
 // one member of an ensemble as seen by the one-launch-per-step kernels
 struct BatchMember {
@@ -159,7 +161,7 @@ struct Context {
     Tune tune_default;            // the shape the context was created with
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    hipEvent_t stage_ev[2] = {nullptr, nullptr};   // copy_to_host chunk completions
+    hipEvent_t stage_ev[8] = {};  // chunk completions of `transfer`
     double last_step_ms = 0.0;
     int device = 0;
     int num_cu = 256;
@@ -185,6 +187,11 @@ struct Context {
     // pinned host staging
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
+
+    // host threads of the bulk transfers (axs_transfer.hip), started on first
+    // use (snapshot_end may be the first, from another host thread)
+    HostPool *pool = nullptr;
+    std::mutex pool_mu;
 
     // asynchronous snapshot (axs_snapshot.hip): device staging copy made on
     // `stream`, device-to-host copy on `copy_stream`
@@ -248,13 +255,23 @@ struct Context {
 int ensure_scratch(Context *c, size_t bytes);
 int ensure_device(Context *c, void **buf, size_t *have, size_t bytes);
 int ensure_pinned(Context *c, size_t bytes);
-// device-to-host copy of `bytes` into a caller's (pageable) buffer through
-// the pinned staging buffer, in chunks whose transfers overlap the host-side
-// copies of the previous chunk; synchronous on return
+// Bulk transfers (axs_transfer.hip).  A segment is L sites of site_bytes each
+// at dev; fn converts sites [lo, lo + n) between their staged bytes and the
+// caller's arrays, on several host threads at once.  Synchronous on return.
+struct Segment {
+    void *dev;
+    size_t site_bytes, L;
+    void (*fn)(char *stage, size_t lo, size_t n, void *arg);
+    void *arg;
+};
+int transfer(Context *c, const Segment *segs, int nsegs, bool to_host);
+// device-to-host copy of `bytes` into a caller's (pageable) buffer
 int copy_to_host(Context *c, void *dst, const void *src, size_t bytes);
-
-// host-side parallel loop over [0, n) in contiguous chunks (std::thread)
-void parallel_for(size_t n, void (*fn)(size_t begin, size_t end, void *arg), void *arg);
+// host-side parallel loop over [0, n) in contiguous pieces on the context's
+// threads (small n: on the calling thread)
+void parallel_for(Context *c, size_t n, void (*fn)(size_t begin, size_t end, void *arg),
+                  void *arg);
+void destroy_pool(Context *c);
 
 // ---------------------------------------------------------------------------
 // launchers (return AXS_OK or an error code)

@@ -205,7 +205,7 @@ int snapshot_end(Context *c, double *out[6], double *tau)
     for (int f = 0; f < 3; ++f) {
         if (!(c->snap_fields & bits[f])) continue;
         Unpack u{src, c->prec == AXS_FP64, out[2 * f], out[2 * f + 1]};
-        if (u.a || u.b) parallel_for((size_t)c->snap_count, unpack_fn, &u);
+        if (u.a || u.b) parallel_for(c, (size_t)c->snap_count, unpack_fn, &u);
         src += per_field;
     }
     if (tau) *tau = c->snap_tau;
