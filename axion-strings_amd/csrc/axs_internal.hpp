@@ -234,6 +234,7 @@ struct Context {
         uint32_t items = 0;
     };
     MultiTables mtab[kMaxDepth + 1];
+    int chunk_key = -1, chunk_planes = 0;     // multi_chunk_planes' last answer
     // blocks of the small 2D lattices' kernel; one lattice's entry by value
     MultiTables blk;
     BatchMember blk_one[2] = {};
@@ -302,8 +303,15 @@ bool multi_shape_built(int D, int W, int R, int prec, int RAD);
 int multi_waves(int flags);
 int multi_waves_of(const Context *c);
 int multi_rows(const Context *c, int N, int D, int W);
-// chunk length cap of the 3D multi-step kernels for tiles TJ x TK
+// chunk lengths of the 3D multi-step kernels for tiles TJ x TK
 int multi_chunk_cap(const Context *c, int TJ, int TK, int H);
+int multi_chunk_planes(Context *c, int TJ, int TK, int H);
+// N planes or rows in equal chunks (to within one) of at most cap
+inline int equal_chunk(int N, int cap)
+{
+    const int n = (N + cap - 1) / cap;
+    return (N + n - 1) / n;
+}
 // largest divisor of N not above cap
 inline int divisor_below(int N, int cap)
 {

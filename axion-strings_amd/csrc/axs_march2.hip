@@ -2,6 +2,10 @@
 // 7-point stencil, and the context-level entry points of the multi-step
 // path: eligibility, work-item tables for ensembles, launches.  Radii 2-4
 // (stencil_setting 1-3) are instantiated in axs_march2_hi.hip.
+#include <math.h>
+
+#include <algorithm>
+
 #include "axs_march2.hpp"
 
 namespace axs {
@@ -40,17 +44,9 @@ int multi_waves(int flags)
 
 int stencil_radius_of(const Context *c) { return c->p.stencil_setting + 1; }
 
-// Chunk of planes per work item (FP32 up to 256, FP64 up to 64, at most
-// half the smallest side) by a cost model: one work-group per CU, every item
-// marches chunk + 2H planes (H = halo), so a pass takes about
-// ceil(items / CUs) * (chunk + 2H) plane steps of one work-group; the
-// cheapest cap wins (ties: the longer chunk).  It reproduces the measured
-// best chunk at every side swept (FP32 depth 4: 256 at 1024^3, 64 at 384^3
-// and 256^3, 32 at 192^3, 8 at 128^3 (depth 3); FP64 depth 3: 64 at 1024^3,
-// 320^3 and 192^3, 32 at 256^3 and 128^3; 64 for both forms' 48-lattice
-// ensemble), where the former rule (fill the chip with at least 3/4
-// (FP32) or 4 (FP64) items per CU) took 8 at FP64 192^3 (1.6x slower)
-// and 128 at FP32 384^3 (1.2x slower).
+// The chunk that a new context's depth rests on (create_impl): of the powers of
+// two (or the side's divisors below them), the chunk of at most 256 (FP32) or 64 (FP64) planes, at most
+// half the smallest side, of least ceil(items / CUs) (chunk + 2H).
 int multi_chunk_cap(const Context *c, int TJ, int TK, int H)
 {
     const bool f32 = c->prec == AXS_FP32;
@@ -71,6 +67,48 @@ int multi_chunk_cap(const Context *c, int TJ, int TK, int H)
             best = cap;
         }
     }
+    return best;
+}
+
+// Most planes per work item of a launch (FP32 up to 256, FP64 up to 64) by a
+// cost model: one work-group per CU, every item marches its chunk + 2H planes
+// (H = halo), so a pass takes about ceil(items / CUs) times the items' mean
+// length; among the choices within 1% of the least, the longest chunk (fewer
+// halo planes read again).  Chunks need not divide the side: a member's planes
+// are dealt in equal chunks of at most this many.  The model keeps the best
+// chunks measured at the sides it was fitted on (FP32 256 at 1024^3, 64 at
+// 256^3; FP64 64 at 1024^3, 640^3 and 192^3); against the longest divisor of
+// the side below a power of two, in us a step: 314^3 FP64 671 -> 256 and FP32
+// 190 -> 73 (divisors 2 and 157), 128^3 FP64 29.2 -> 22.7, 256^3 FP64 150.6 ->
+// 145, 64^3 FP64 10.1 -> 7.8, 320^3 FP32 70 -> 60, 256^3 FP32 sixth order 127 ->
+// 103, the 48-lattice FP32 ensemble (128-plane chunks for 64) 777 -> 734.
+int multi_chunk_planes(Context *c, int TJ, int TK, int H)
+{
+    const int key = (TJ * 128 + TK) * 64 + H;
+    if (c->chunk_key == key) return c->chunk_planes;
+    const int most = (c->prec == AXS_FP32) ? 256 : 64;
+    const double cus = c->num_cu > 0 ? c->num_cu : 1;
+    auto cost_of = [&](int cap) {
+        double items = 0.0, planes = 0.0;
+        for (const Member &m : c->members) {
+            const int ci = equal_chunk(m.N, cap);
+            const double n = (double)((m.N + TJ - 1) / TJ) * (double)((m.N + TK - 1) / TK) *
+                             (double)((m.N + ci - 1) / ci);
+            items += n;
+            planes += n * (double)(ci + 2 * H);
+        }
+        return ceil(items / cus) * (planes / items);
+    };
+    double least = 1e300;
+    for (int cap = 4; cap <= most; ++cap) least = std::min(least, cost_of(cap));
+    int best = 4;
+    for (int cap = most; cap >= 4; --cap)
+        if (cost_of(cap) <= 1.01 * least) {
+            best = cap;
+            break;
+        }
+    c->chunk_key = key;
+    c->chunk_planes = best;
     return best;
 }
 
@@ -242,7 +280,7 @@ int prepare_multi_batch(Context *c, int D)
         b.nTj = (m.N + TJ - 1) / TJ;
         b.nTk = (m.N + TK - 1) / TK;
         b.CI = multi_chunk(c, m.N, TJ, TK, D * RAD);
-        items += (uint32_t)b.nTj * b.nTk * (m.N / b.CI);
+        items += (uint32_t)b.nTj * b.nTk * (uint32_t)((m.N + b.CI - 1) / b.CI);
         for (int h = 0; h < 2; ++h) {
             for (int a = 0; a < 3; ++a) {
                 b.in[a] = m.state[h][a];

@@ -124,9 +124,10 @@ template <class T, int D, int W, int R, int RAD>
 using TBLds = T[D][2][(W * R + 2 * RAD) * kTBW];
 
 // One work-group: tile (tj, tk) of the lattice of side N, planes
-// [ch*CI, ch*CI + CI).
+// [ch*chunk, ch*chunk + chunk), fewer in the last chunk where they do not
+// divide N.
 template <class Tr, int D, int W, int R, int RAD, bool PF>
-__device__ __forceinline__ void marchd_tile(const int N, const int CI, const int tj, const int tk,
+__device__ __forceinline__ void marchd_tile(const int N, const int chunk, const int tj, const int tk,
                                             const int ch, const typename Tr::In &in,
                                             const typename Tr::Out &out,
                                             const LevelScalars<typename Tr::Sc, D> &sc,
@@ -148,7 +149,8 @@ __device__ __forceinline__ void marchd_tile(const int N, const int CI, const int
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t NN = (uint32_t)N * (uint32_t)N;
-    const int j0 = tj * TJ, k0 = tk * TK + K0, i0 = ch * CI;
+    const int j0 = tj * TJ, k0 = tk * TK + K0, i0 = ch * chunk;
+    const int CI = (N - i0 < chunk) ? N - i0 : chunk;
 
     // column of this lane, wrapped: -HK <= k0 - HK + lane < 2N for N >= 64;
     // it is written if it lies in the lanes' output range and in the first
@@ -422,12 +424,13 @@ marchd_batch_kernel(const BatchMember *__restrict__ mem, int n_members, uint32_t
 }
 
 // planes per chunk of a member of side N, tiles TJ x TK: the configured
-// count if it divides N, else the ensemble-wide choice of multi_chunk_cap
-inline int multi_chunk(const Context *c, int N, int TJ, int TK, int H)
+// count if it divides N, else chunks equal to within a plane, of at most the
+// context-wide choice of multi_chunk_planes
+inline int multi_chunk(Context *c, int N, int TJ, int TK, int H)
 {
     const int ci = c->tune.ci32;
     if (ci > 0 && N % ci == 0) return ci;
-    return divisor_below(N, multi_chunk_cap(c, TJ, TK, H));
+    return equal_chunk(N, multi_chunk_planes(c, TJ, TK, H));
 }
 
 template <class Sc>
@@ -458,7 +461,7 @@ struct SingleLaunch {
         g.nTj = (N + TJ - 1) / TJ;
         g.nTk = (N + TK - 1) / TK;
         g.CI = multi_chunk(c, N, TJ, TK, D * RAD);
-        const uint32_t nb = (uint32_t)g.nTj * (uint32_t)g.nTk * (uint32_t)(N / g.CI);
+        const uint32_t nb = (uint32_t)g.nTj * (uint32_t)g.nTk * (uint32_t)((N + g.CI - 1) / g.CI);
         tile_order<Tr>(g);
         if (pf)
             hipLaunchKernelGGL((marchd_kernel<Tr, D, W, R, RAD, true>), dim3(nb), dim3(64 * W), 0,

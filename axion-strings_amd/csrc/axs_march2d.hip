@@ -49,15 +49,6 @@ static int pick_cap(const Context *c, int TI, int H)
     return best;
 }
 
-// rows per chunk of a lattice of side N for a choice of `cap` rows: the
-// chunks are made equal to within a row (the last one is shorter where they
-// do not divide N)
-static int chunk_rows(int N, int cap)
-{
-    const int n = (N + cap - 1) / cap;
-    return (N + n - 1) / n;
-}
-
 int prepare_march2d_items(Context *c, int D)
 {
     if (D < 1) return AXS_OK;
@@ -77,7 +68,7 @@ int prepare_march2d_items(Context *c, int D)
         b.nTj = (m.N + TI - 1) / TI;       // strips
         b.nTk = 1;
         const int cfg = c->tune.ci32;      // rows per chunk
-        b.CI = (cfg > 0 && m.N % cfg == 0) ? cfg : chunk_rows(m.N, cap);
+        b.CI = (cfg > 0 && m.N % cfg == 0) ? cfg : equal_chunk(m.N, cap);   // last one shorter
         items += (uint32_t)b.nTj * (uint32_t)((m.N + b.CI - 1) / b.CI);
         for (int h = 0; h < 2; ++h) {
             for (int a = 0; a < 3; ++a) {
