@@ -722,9 +722,9 @@ int axs_step(axs_ctx *ctx, int64_t nsteps)
             return AXS_ERR_STATE;
         }
     if (nsteps == 0) return AXS_OK;
-    const int blk = block2d_depth(c);
+    const int blk = block_depth(c);
     if (blk > 0)
-        AXS_TRY(prepare_block2d(c));
+        AXS_TRY(prepare_blocks(c));
     else
         AXS_TRY(prepare_batch(c));
     const double dt = (double)c->p.time_step;
@@ -761,7 +761,7 @@ int axs_step(axs_ctx *ctx, int64_t nsteps)
                 t = t + dt;                               // the same sequence of sums
                 ss[l] = make_scalars(c->p, t);
             }
-            rc = (blk > 0) ? launch_block2d(c, ss, d) : launch_multi_steps(c, ss, d);
+            rc = (blk > 0) ? launch_blocks(c, ss, d) : launch_multi_steps(c, ss, d);
             if (rc == AXS_OK) {
                 c->tau = t;
                 ++launches;

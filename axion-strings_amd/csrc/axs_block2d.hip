@@ -228,12 +228,11 @@ int block2d_depth(const Context *c)
     return blk_depth(RAD);
 }
 
-int prepare_block2d(Context *c)
+// member tables of the block kernels, for blocks of TI columns and TJ rows (2D)
+// or TI^3 sites (3D)
+int block_tables(Context *c, int TI, int TJ, int key)
 {
     Context::MultiTables &mt = c->blk;
-    const int RAD = stencil_radius_of(c), R = block2d_rows(c);
-    if (mt.key == R) return AXS_OK;
-    const int TI = blk_cols(RAD), TJ = blk_rows(RAD, R);
     std::vector<BatchMember> tab[2];
     uint32_t items = 0;
     for (const Member &m : c->members) {
@@ -243,7 +242,7 @@ int prepare_block2d(Context *c)
         b.item_begin = items;
         b.nTj = (m.N + TJ - 1) / TJ;
         b.nTk = (m.N + TI - 1) / TI;
-        items += (uint32_t)b.nTj * (uint32_t)b.nTk;
+        items += (uint32_t)b.nTj * (uint32_t)b.nTk * (c->nd == 3 ? (uint32_t)b.nTj : 1u);
         for (int h = 0; h < 2; ++h) {
             for (int a = 0; a < 3; ++a) {
                 b.in[a] = m.state[h][a];
@@ -263,8 +262,30 @@ int prepare_block2d(Context *c)
     }
     if (c->members.size() > 1) AXS_HIP_TRY(hipStreamSynchronize(c->stream));
     mt.items = items;
-    mt.key = R;
+    mt.key = key;
     return AXS_OK;
+}
+
+int prepare_block2d(Context *c)
+{
+    const int RAD = stencil_radius_of(c), R = block2d_rows(c);
+    if (c->blk.key == R) return AXS_OK;
+    return block_tables(c, blk_cols(RAD), blk_rows(RAD, R), R);
+}
+
+int block_depth(const Context *c)
+{
+    return (c->nd == 2) ? block2d_depth(c) : block3d_depth(c);
+}
+
+int prepare_blocks(Context *c)
+{
+    return (c->nd == 2) ? prepare_block2d(c) : prepare_block3d(c);
+}
+
+int launch_blocks(Context *c, const StepScalars *s, int d)
+{
+    return (c->nd == 2) ? launch_block2d(c, s, d) : launch_block3d(c, s, d);
 }
 
 template <class Tr, int RAD, int R>

@@ -235,7 +235,7 @@ struct Context {
     };
     MultiTables mtab[kMaxDepth + 1];
     int chunk_key = -1, chunk_planes = 0;     // multi_chunk_planes' last answer
-    // blocks of the small 2D lattices' kernel; one lattice's entry by value
+    // blocks of the small lattices' kernels; one lattice's entry by value
     MultiTables blk;
     BatchMember blk_one[2] = {};
     // string finder results of the last call (ballot words, block counts,
@@ -335,11 +335,17 @@ int prepare_march2d_items(Context *c, int D);
 int launch_march2d(Context *c, int src, const StepScalars *s, int depth);
 // higher-order stencils (radius 2-4), 2D (axs_march2d_hi.hip)
 int launch_march2d_high_order(Context *c, int src, const StepScalars *s, int depth, bool pf);
-// small 2D lattices (axs_block2d.hip): most steps of one pass, or 0 where
-// the strip kernels run
+// small lattices (axs_block2d.hip, axs_block3d.hip): most steps of one pass, or
+// 0 where the strip and marching kernels run; d <= block_depth steps in one pass
+int block_depth(const Context *c);
+int prepare_blocks(Context *c);
+int launch_blocks(Context *c, const StepScalars *s, int d);
 int block2d_depth(const Context *c);
-int prepare_block2d(Context *c);
+int block3d_depth(const Context *c);
+int block_tables(Context *c, int TI, int TJ, int key);
+int prepare_block3d(Context *c);
 int launch_block2d(Context *c, const StepScalars *s, int d);
+int launch_block3d(Context *c, const StepScalars *s, int d);
 // field-rescaled step with the spectral Laplacian, one member
 int run_spectral_step(Context *c, Member &m, int src, int dst, const StepScalars &s);
 // Laplacian of the current field (AXS_LAPLACIAN_*) into host arrays

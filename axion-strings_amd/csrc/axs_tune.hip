@@ -90,9 +90,9 @@ void append_file_cache(const std::string &key, const Tune &t, double ms)
 // time `trials` steps of the current configuration without changing state
 int time_trial(Context *c, int trials, double *ms)
 {
-    const int blk = block2d_depth(c);     // the automatic shape of a small 2D lattice
+    const int blk = block_depth(c);     // the automatic shape of a small lattice
     if (blk > 0)
-        AXS_TRY(prepare_block2d(c));
+        AXS_TRY(prepare_blocks(c));
     else
         AXS_TRY(prepare_batch(c));
     const int cur0 = c->cur;
@@ -107,7 +107,7 @@ int time_trial(Context *c, int trials, double *ms)
     const StepScalars &s = ss[0];
     // one trial = one launch of one or several steps
     auto one = [&]() {
-        if (blk > 0) return launch_block2d(c, ss, blk);
+        if (blk > 0) return launch_blocks(c, ss, blk);
         return depth >= 1 ? launch_multi_steps(c, ss, depth) : launch_step(c, s);
     };
     AXS_TRY(one());                             // warm-up (code objects, caches)
@@ -280,10 +280,10 @@ int run_autotune(Context *c, int trials, double *best_ms)
     }
     for (Tune &t : cands) t.configured = true;
     const Tune saved = c->tune;
-    // the block kernel of small 2D lattices runs in the context's own shape,
+    // the block kernels of small lattices run in the context's own shape,
     // reported as the shape that runs without it
     c->tune = c->tune_default;
-    if (block2d_depth(c) > 0) {
+    if (block_depth(c) > 0) {
         Tune u = c->tune_default;
         u.kernel = strips_ok ? AXS_KERNEL_MARCH : AXS_KERNEL_SIMPLE;
         cands.push_back(u);

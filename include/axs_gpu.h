@@ -286,7 +286,7 @@ typedef struct axs_kernel_config {
                      4), else end with shallower multi-step passes where
                      built, else with one-step launches; every split gives
                      the same bits.  Small 2D lattices and sides below 64
-                     run up to six steps per pass on a kernel of their own,
+                     run up to six steps per pass on kernels of their own,
                      with the same bits, until a configuration is set.      */
     int flags;    /* AXS_MARCH_* bits                                       */
 } axs_kernel_config;
