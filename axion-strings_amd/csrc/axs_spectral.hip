@@ -28,9 +28,9 @@ struct SpecPlan {
     rocfft_execution_info fwd_info = nullptr, bwd_info = nullptr;
     void *work = nullptr;
     size_t work_bytes = 0;
-    double *real = nullptr;     // one real component (transform input/output)
     double *spec = nullptr;     // half spectrum, interleaved complex
-    double *lap = nullptr;      // two Laplacian components, L doubles each
+    double *lap = nullptr;      // two real components, L doubles each: the field,
+                                // then its Laplacian times the length
     double *ktab = nullptr;     // k[i], i = 0..N-1 (s_integrate.cpp:192, :242)
     ~SpecPlan()
     {
@@ -38,7 +38,7 @@ struct SpecPlan {
         if (bwd) rocfft_plan_destroy(bwd);
         if (fwd_info) rocfft_execution_info_destroy(fwd_info);
         if (bwd_info) rocfft_execution_info_destroy(bwd_info);
-        for (void *p : {(void *)work, (void *)real, (void *)spec, (void *)lap, (void *)ktab})
+        for (void *p : {(void *)work, (void *)spec, (void *)lap, (void *)ktab})
             if (p) (void)hipFree(p);
     }
 };
@@ -83,8 +83,7 @@ static int get_spec_plan(Context *c, int N, SpecPlan **out)
         return AXS_ERR_FFT;
     }
     p->work_bytes = wf > wb ? wf : wb;
-    hipError_t e = hipMalloc(&p->real, L * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&p->spec, half * 2 * sizeof(double));
+    hipError_t e = hipMalloc(&p->spec, half * 2 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&p->lap, 2 * L * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&p->ktab, (size_t)N * sizeof(double));
     if (e == hipSuccess && p->work_bytes) e = hipMalloc(&p->work, p->work_bytes);
@@ -171,27 +170,22 @@ minus_k2_kernel(int N, uint32_t nhalf, const double *__restrict__ k, double *__r
 
 // ret = data / length (:230-231)
 __global__ void __launch_bounds__(256)
-scale_kernel(uint32_t L, const double *__restrict__ x, double len, double *__restrict__ y)
+scale_kernel(uint32_t L, double *__restrict__ x, double len)
 {
     uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m < L) y[m] = x[m] / len;
+    if (m < L) x[m] = x[m] / len;
 }
 
-// spectral Laplacian of comp of the field into lap (device, L doubles)
-template <class P>
-static int spectral_component(Context *c, SpecPlan *sp, uint32_t L, const P &phi, int comp,
-                              double *lap)
+// spectral Laplacian of the real component at x (device, L doubles), in place,
+// not yet divided by the length
+static int spectral_component(Context *c, SpecPlan *sp, uint32_t L, double *x)
 {
-    const unsigned grid = (L + 255) / 256;
-    hipLaunchKernelGGL(component_kernel<P>, dim3(grid), dim3(256), 0, c->stream, L, phi, comp,
-                       sp->real);
-    AXS_HIP_TRY(hipGetLastError());
     if (rocfft_execution_info_set_stream(sp->fwd_info, c->stream) != rocfft_status_success ||
         rocfft_execution_info_set_stream(sp->bwd_info, c->stream) != rocfft_status_success) {
         set_error("rocfft_execution_info_set_stream failed");
         return AXS_ERR_FFT;
     }
-    void *in[1] = {sp->real}, *out[1] = {sp->spec};
+    void *in[1] = {x}, *out[1] = {sp->spec};
     if (rocfft_execute(sp->fwd, in, out, sp->fwd_info) != rocfft_status_success) {
         set_error("rocfft forward transform failed");
         return AXS_ERR_FFT;
@@ -201,21 +195,21 @@ static int spectral_component(Context *c, SpecPlan *sp, uint32_t L, const P &phi
     hipLaunchKernelGGL(kk, dim3((nhalf + 255) / 256), dim3(256), 0, c->stream, sp->N, nhalf,
                        sp->ktab, sp->spec);
     AXS_HIP_TRY(hipGetLastError());
-    void *bin[1] = {sp->spec}, *bout[1] = {sp->real};
+    void *bin[1] = {sp->spec}, *bout[1] = {x};
     if (rocfft_execute(sp->bwd, bin, bout, sp->bwd_info) != rocfft_status_success) {
         set_error("rocfft inverse transform failed");
         return AXS_ERR_FFT;
     }
-    hipLaunchKernelGGL(scale_kernel, dim3(grid), dim3(256), 0, c->stream, L, sp->real, (double)L,
-                       lap);
-    AXS_HIP_TRY(hipGetLastError());
     return AXS_OK;
 }
 
-// drift of the field-rescaled form (s_integrate.cpp:313-314) into out.phi
+// drift of the field-rescaled form (s_integrate.cpp:313-314) into out.phi, and
+// each component on its own for the transforms (a pass per component read the
+// pairs back for that: 69 us of 1640 each at 256^3)
 __global__ void __launch_bounds__(256)
 spectral_drift_kernel(uint32_t L, const dvec2 *__restrict__ phi, const dvec2 *__restrict__ vel,
-                      const dvec2 *__restrict__ ker, dvec2 *__restrict__ xo, double dt)
+                      const dvec2 *__restrict__ ker, dvec2 *__restrict__ xo,
+                      double *__restrict__ x1, double *__restrict__ x2, double dt)
 {
     uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= L) return;
@@ -223,22 +217,25 @@ spectral_drift_kernel(uint32_t L, const dvec2 *__restrict__ phi, const dvec2 *__
     x.x = p.x + dt * (v.x + 0.5 * k.x * dt);
     x.y = p.y + dt * (v.y + 0.5 * k.y * dt);
     xo[m] = x;
+    x1[m] = x.x;
+    x2[m] = x.y;
 }
 
-// ker_next = Laplacian, then the potential (:331-335), kick (:337-341)
+// ker_next = Laplacian (divided by the length here, :230-231), then the
+// potential (:331-335), kick (:337-341)
 __global__ void __launch_bounds__(256)
 spectral_finish_kernel(uint32_t L, const dvec2 *__restrict__ x, const double *__restrict__ lap1,
                        const double *__restrict__ lap2, const dvec2 *__restrict__ vel,
                        const dvec2 *__restrict__ ker, dvec2 *__restrict__ vo,
-                       dvec2 *__restrict__ ko, StepScalars s)
+                       dvec2 *__restrict__ ko, StepScalars s, double len)
 {
     uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= L) return;
     dvec2 xv = x[m];
     double S = xv.x * xv.x + xv.y * xv.y - s.tau2 + s.T03;
     dvec2 kn, vn, kc = ker[m], vc = vel[m];
-    kn.x = lap1[m] + s.cl * xv.x * S;
-    kn.y = lap2[m] + s.cl * xv.y * S;
+    kn.x = lap1[m] / len + s.cl * xv.x * S;
+    kn.y = lap2[m] / len + s.cl * xv.y * S;
     vn.x = vc.x + 0.5 * (kc.x + kn.x) * s.dt;
     vn.y = vc.y + 0.5 * (kc.y + kn.y) * s.dt;
     vo[m] = vn;
@@ -255,14 +252,13 @@ int run_spectral_step(Context *c, Member &m, int src, int dst, const StepScalars
                 *ker = (const dvec2 *)m.state[src][KER];
     dvec2 *xo = (dvec2 *)m.state[dst][PHI];
     hipLaunchKernelGGL(spectral_drift_kernel, dim3(grid), dim3(256), 0, c->stream, L, phi, vel,
-                       ker, xo, s.dt);
+                       ker, xo, sp->lap, sp->lap + L, s.dt);
     AXS_HIP_TRY(hipGetLastError());
-    PhiF64 x{xo};
-    AXS_TRY(spectral_component(c, sp, L, x, 0, sp->lap));
-    AXS_TRY(spectral_component(c, sp, L, x, 1, sp->lap + L));
+    AXS_TRY(spectral_component(c, sp, L, sp->lap));
+    AXS_TRY(spectral_component(c, sp, L, sp->lap + L));
     hipLaunchKernelGGL(spectral_finish_kernel, dim3(grid), dim3(256), 0, c->stream, L, xo,
                        sp->lap, sp->lap + L, vel, ker, (dvec2 *)m.state[dst][VEL],
-                       (dvec2 *)m.state[dst][KER], s);
+                       (dvec2 *)m.state[dst][KER], s, (double)L);
     AXS_HIP_TRY(hipGetLastError());
     return AXS_OK;
 }
@@ -303,14 +299,20 @@ int run_laplacian(Context *c, Member &m, int mode, double *h1, double *h2)
     AXS_TRY(get_spec_plan(c, m.N, &sp));     // its buffers hold the result either way
     const uint32_t L = (uint32_t)m.L;
     if (mode == AXS_LAPLACIAN_SPECTRAL) {
-        if (c->prec == AXS_FP64) {
-            PhiF64 x{(const dvec2 *)fv.phi};
-            AXS_TRY(spectral_component(c, sp, L, x, 0, sp->lap));
-            AXS_TRY(spectral_component(c, sp, L, x, 1, sp->lap + L));
-        } else {
-            PhiF32 x{(const fvec4 *)fv.phi};
-            AXS_TRY(spectral_component(c, sp, L, x, 0, sp->lap));
-            AXS_TRY(spectral_component(c, sp, L, x, 1, sp->lap + L));
+        const unsigned grid = (L + 255) / 256;
+        for (int comp = 0; comp < 2; ++comp) {
+            double *x = sp->lap + (size_t)comp * L;
+            if (c->prec == AXS_FP64)
+                hipLaunchKernelGGL(component_kernel<PhiF64>, dim3(grid), dim3(256), 0, c->stream,
+                                   L, PhiF64{(const dvec2 *)fv.phi}, comp, x);
+            else
+                hipLaunchKernelGGL(component_kernel<PhiF32>, dim3(grid), dim3(256), 0, c->stream,
+                                   L, PhiF32{(const fvec4 *)fv.phi}, comp, x);
+            AXS_HIP_TRY(hipGetLastError());
+            AXS_TRY(spectral_component(c, sp, L, x));
+            hipLaunchKernelGGL(scale_kernel, dim3(grid), dim3(256), 0, c->stream, L, x,
+                               (double)L);
+            AXS_HIP_TRY(hipGetLastError());
         }
     } else {
         // the field-rescaled stencil operator: alpha = 1.0f / pow_2(dx)
