@@ -17,9 +17,10 @@
 // Each level keeps x_l of planes q-RAD .. q+RAD-1 in registers (plane
 // q+RAD is the value the level below has just produced) -- the i neighbours
 // -- and the own data of planes q .. q+RAD-1 (produced RAD planes before
-// they are used); x_l of plane q sits in one LDS plane per level for the j
-// and k neighbours, written after a barrier that ends the plane's reads and
-// read after a second barrier.  The Laplacian sums in the one-step kernels'
+// they are used); x_l of plane q sits in an LDS plane per level for the j
+// and k neighbours (two sets in turn where they fit, one barrier a plane; else
+// one, written after a barrier that ends the plane's reads and read after a
+// second: kTwoSets).  The Laplacian sums in the one-step kernels'
 // order -- the form's centre term, then for each distance m: +-i, +-j,
 // +-k, each times the stencil coefficient -- with the forms' expressions,
 // so a pass is bit-identical to D one-step launches.  Tiles at the lattice
@@ -117,21 +118,39 @@ __device__ __forceinline__ void tile_of(uint32_t t, const TBGeom &g, int &tj, in
     tk = (int)(loc / h);
 }
 
+// LDS sets of the levels' planes.  Two, where they fit: the next plane goes to
+// the other set, and one barrier a plane orders both.  One: a barrier before the
+// writes and one after.  Two are faster on every lattice tried (us a step: FP32
+// 512^3 260 -> 245, 640^3 460 -> 441, 896^3 1187 -> 1148, the 48-lattice ensemble
+// 720 -> 712; FP64 128^3 22.1 -> 21.1, 256^3 147 -> 143, 640^3 1.82 -> 1.74 ms,
+// 1024^3 7.17 -> 7.05 ms) but one: FP32 rows of a whole number of 16 KiB
+// (1024^3), whose lines of one column fall on the same memory channels; there
+// the freer waves spread the work-groups' planes apart, 1.77 -> 1.86 ms.
+template <class T, int D, int W, int R, int RAD>
+constexpr bool kTwoSets = 2 * D * 2 * (W * R + 2 * RAD) * kTBW * (int)sizeof(T) <= 160 * 1024;
+template <class Tr, int D, int W, int R, int RAD>
+inline bool two_sets(int N)
+{
+    using T = typename Tr::T;
+    if (!kTwoSets<T, D, W, R, RAD>) return false;
+    return !std::is_same<T, float>::value || (size_t)N * 16 % 16384 != 0;
+}
+
 // x_l of the plane level l works on: the ER loaded rows plus RAD padding
 // rows above and below, so that the neighbour reads of the rim rows and
 // lanes stay inside the array (their values are never used)
-template <class T, int D, int W, int R, int RAD>
-using TBLds = T[D][2][(W * R + 2 * RAD) * kTBW];
+template <class T, int D, int W, int R, int RAD, int SETS>
+using TBLds = T[SETS][D][2][(W * R + 2 * RAD) * kTBW];
 
 // One work-group: tile (tj, tk) of the lattice of side N, planes
 // [ch*chunk, ch*chunk + chunk), fewer in the last chunk where they do not
 // divide N.
-template <class Tr, int D, int W, int R, int RAD, bool PF>
+template <class Tr, int D, int W, int R, int RAD, bool PF, int SETS>
 __device__ __forceinline__ void marchd_tile(const int N, const int chunk, const int tj, const int tk,
                                             const int ch, const typename Tr::In &in,
                                             const typename Tr::Out &out,
                                             const LevelScalars<typename Tr::Sc, D> &sc,
-                                            TBLds<typename Tr::T, D, W, R, RAD> &X)
+                                            TBLds<typename Tr::T, D, W, R, RAD, SETS> &X)
 {
     using T = typename Tr::T;
     using Own = typename Tr::Own;
@@ -213,6 +232,7 @@ __device__ __forceinline__ void marchd_tile(const int N, const int chunk, const 
     const typename Tr::Vc vc = Tr::vconst(sc.s[0]);
 
     if (PF) load(i0 - H, pf);
+    int set = 0;
     auto plane_step = [&](const int it) __attribute__((always_inline)) {
         const int i = i0 + it;
         // level 0: plane i+H
@@ -232,7 +252,7 @@ __device__ __forceinline__ void marchd_tile(const int N, const int chunk, const 
         for (int l = 1; l <= D; ++l) {
             const typename Tr::Sc &s = sc.s[l - 1];
             const typename Tr::Sc &sn = sc.s[l < D ? l : D - 1];
-            const T *L1 = X[l - 1][0], *L2 = X[l - 1][1];
+            const T *L1 = X[set][l - 1][0], *L2 = X[set][l - 1][1];
             // level l computes from the first plane on: until x_l of planes
             // q-RAD .. q+RAD exist (it >= 2 RAD (l - D)) its results are
             // unused -- they leave the ring of level l+1 before it fills
@@ -342,15 +362,18 @@ __device__ __forceinline__ void marchd_tile(const int N, const int chunk, const 
                 }
             }
         }
-        __syncthreads();   // every read of this plane's LDS values is done
+        if constexpr (SETS == 2)
+            set ^= 1;          // this plane's reads end before the next barrier
+        else
+            __syncthreads();   // every read of this plane's LDS values is done
         // each level's next plane (q+1) is now the middle of its ring
 #pragma unroll
         for (int l = 0; l < D; ++l) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int o = (erow[r] + RAD) * kTBW + lane;
-                X[l][0][o] = ring[l][RAD][r][0];
-                X[l][1][o] = ring[l][RAD][r][1];
+                X[set][l][0][o] = ring[l][RAD][r][0];
+                X[set][l][1][o] = ring[l][RAD][r][1];
             }
         }
         __syncthreads();   // the next plane's values are visible
@@ -366,18 +389,18 @@ __device__ __forceinline__ void marchd_tile(const int N, const int chunk, const 
     for (; it < CI; ++it) plane_step(it);
 }
 
-template <class Tr, int D, int W, int R, int RAD, bool PF>
+template <class Tr, int D, int W, int R, int RAD, bool PF, int SETS>
 __global__ void __launch_bounds__(64 * W)
 marchd_kernel(TBGeom g, typename Tr::In in, typename Tr::Out out,
               LevelScalars<typename Tr::Sc, D> sc)
 {
-    __shared__ TBLds<typename Tr::T, D, W, R, RAD> X;
+    __shared__ TBLds<typename Tr::T, D, W, R, RAD, SETS> X;
     const uint32_t b = g.xcd ? xcd_order(blockIdx.x, gridDim.x) : blockIdx.x;
     const uint32_t layer = (uint32_t)g.nTj * (uint32_t)g.nTk;
     int tj, tk;
     tile_of(b % layer, g, tj, tk);
     const int ch = (int)(b / layer);
-    marchd_tile<Tr, D, W, R, RAD, PF>(g.N, g.CI, tj, tk, ch, in, out, sc, X);
+    marchd_tile<Tr, D, W, R, RAD, PF, SETS>(g.N, g.CI, tj, tk, ch, in, out, sc, X);
 }
 
 // the form's array views from a member-table entry (device) or a member (host)
@@ -400,14 +423,14 @@ __host__ __device__ __forceinline__ typename Tr::Out form_out(void *const *p)
 
 // Ensemble form: one persistent launch for every member.  Work items are
 // the (member, tile, chunk) triples, members in order, tiles k fastest;
-// work-group b takes items b, b + gridDim.x, ...  The first barrier of a
-// tile orders its LDS writes after the previous tile's reads.
-template <class Tr, int D, int W, int R, int RAD, bool PF>
+// work-group b takes items b, b + gridDim.x, ...  The barrier that ends a
+// tile's last plane orders the next tile's LDS writes after its reads.
+template <class Tr, int D, int W, int R, int RAD, bool PF, int SETS>
 __global__ void __launch_bounds__(64 * W)
 marchd_batch_kernel(const BatchMember *__restrict__ mem, int n_members, uint32_t n_items,
                     LevelScalars<typename Tr::Sc, D> sc)
 {
-    __shared__ TBLds<typename Tr::T, D, W, R, RAD> X;
+    __shared__ TBLds<typename Tr::T, D, W, R, RAD, SETS> X;
     for (uint32_t item = blockIdx.x; item < n_items; item += gridDim.x) {
         int lo = 0, hi = n_members - 1;        // last member starting at or before item
         while (lo < hi) {
@@ -423,8 +446,8 @@ marchd_batch_kernel(const BatchMember *__restrict__ mem, int n_members, uint32_t
         t /= (uint32_t)m.nTk;
         const int tj = (int)(t % (uint32_t)m.nTj);
         const int ch = (int)(t / (uint32_t)m.nTj);
-        marchd_tile<Tr, D, W, R, RAD, PF>(m.N, m.CI, tj, tk, ch, form_in<Tr>(m.in),
-                                          form_out<Tr>(m.out), sc, X);
+        marchd_tile<Tr, D, W, R, RAD, PF, SETS>(m.N, m.CI, tj, tk, ch, form_in<Tr>(m.in),
+                                                form_out<Tr>(m.out), sc, X);
     }
 }
 
@@ -468,13 +491,25 @@ struct SingleLaunch {
         g.CI = multi_chunk(c, N, TJ, TK, D * RAD);
         const uint32_t nb = (uint32_t)g.nTj * (uint32_t)g.nTk * (uint32_t)((N + g.CI - 1) / g.CI);
         tile_order<Tr>(g);
-        if (pf)
-            hipLaunchKernelGGL((marchd_kernel<Tr, D, W, R, RAD, true>), dim3(nb), dim3(64 * W), 0,
-                               c->stream, g, in, out, sc);
-        else
-            hipLaunchKernelGGL((marchd_kernel<Tr, D, W, R, RAD, false>), dim3(nb), dim3(64 * W),
-                               0, c->stream, g, in, out, sc);
+        if constexpr (kTwoSets<typename Tr::T, D, W, R, RAD>) {
+            if (two_sets<Tr, D, W, R, RAD>(N)) {
+                launch<W, R, 2>(nb, g);
+                return AXS_OK;
+            }
+        }
+        if constexpr (std::is_same<Tr, F32Form>::value || !kTwoSets<typename Tr::T, D, W, R, RAD>)
+            launch<W, R, 1>(nb, g);
         return AXS_OK;
+    }
+    template <int W, int R, int SETS>
+    void launch(uint32_t nb, const TBGeom &g)
+    {
+        if (pf)
+            hipLaunchKernelGGL((marchd_kernel<Tr, D, W, R, RAD, true, SETS>), dim3(nb),
+                               dim3(64 * W), 0, c->stream, g, in, out, sc);
+        else
+            hipLaunchKernelGGL((marchd_kernel<Tr, D, W, R, RAD, false, SETS>), dim3(nb),
+                               dim3(64 * W), 0, c->stream, g, in, out, sc);
     }
 };
 
@@ -487,8 +522,20 @@ struct BatchLaunch {
     template <int W, int R>
     int run()
     {
-        auto kern = pf ? marchd_batch_kernel<Tr, D, W, R, RAD, true>
-                       : marchd_batch_kernel<Tr, D, W, R, RAD, false>;
+        if constexpr (kTwoSets<typename Tr::T, D, W, R, RAD>) {
+            bool two = true;
+            for (const Member &m : c->members) two = two && two_sets<Tr, D, W, R, RAD>(m.N);
+            if (two) return launch<W, R, 2>();
+        }
+        if constexpr (std::is_same<Tr, F32Form>::value || !kTwoSets<typename Tr::T, D, W, R, RAD>)
+            return launch<W, R, 1>();
+        return AXS_OK;
+    }
+    template <int W, int R, int SETS>
+    int launch()
+    {
+        auto kern = pf ? marchd_batch_kernel<Tr, D, W, R, RAD, true, SETS>
+                       : marchd_batch_kernel<Tr, D, W, R, RAD, false, SETS>;
         int per_cu = 0;
         AXS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * W, 0));
         const uint32_t cap = (uint32_t)c->num_cu * (uint32_t)(per_cu > 0 ? per_cu : 1);
