@@ -6,9 +6,9 @@
 // The reference multiplies the field by (-1)^(i+j+k) and takes a complex
 // forward FFT of the whole N^d array, so that array index i corresponds to
 // the signed frequency i - N/2.  The shift only relabels modes; here the
-// unshifted field goes through a rocFFT real-to-complex transform (half the
-// spectrum, half the memory) and each stored mode (fi, fj, fz >= 0) stands
-// for itself and, when 0 < fz < N/2, for its Hermitian partner -k with the
+// unshifted field goes through a real-to-complex transform (half the spectrum,
+// half the memory; our own, or rocFFT where own_fft_ok and any_fft_ok refuse)
+// and each stored mode (fi, fj, fz >= 0) stands for itself and, when 0 < fz < N/2, for its Hermitian partner -k with the
 // same |F|^2 and |k| (weight 2).
 //
 // Binning is done per bin rather than per mode: a bin is a range [lo, hi)
@@ -32,7 +32,7 @@ namespace axs {
 
 struct FftPlan {
     int N = 0, nd = 0, batch = 1;
-    bool own = false;           // the transform of our own (power-of-two sides)
+    bool own = false;           // a transform of our own
     rocfft_plan plan = nullptr;
     rocfft_execution_info info = nullptr;
     void *work = nullptr;
@@ -932,6 +932,479 @@ fft_bin_kernel(const double2 *__restrict__ y, const double2 *__restrict__ tw, in
     }
 }
 
+// ---------------------------------------------------------------------------
+// Other sides: the same passes with the side at run time, for every even N
+// whose half has no prime factor above 7 (any_fft_ok).  A row's transform is a
+// list of Stockham stages of radix 16, 8, 7, 5, 4, 3 and 2, each the code below
+// for that radix: a thread reads its butterflies of the stage into registers,
+// and writes them after a barrier.
+//
+// Bound: latency.  The LDS of a group's rows leaves two work-groups a CU in the Z
+// pass and one in Y, whose loads, stages and stores follow one another; at 400^3
+// the three passes' 3 GB would take 0.6 ms.  So a thread's loads are in flight
+// together (clamped to the last row, not guarded) and the twiddles lie in LDS
+// (any_tw), the two together 1634 -> 1173 us at 400^3; and a small lattice's rows
+// are spread over all CUs (any_group: 113 -> 75 us at 48^3).  Radices 6, 10, 12, 14 and 15 as two coprime factors, which save
+// a stage of three or four at some sides, gained 7 to 14 % at 300^3, 500^3 and
+// 900^3, nothing at 200^3, 320^3 and 400^3, and lost 3 % at 640^3: not taken.
+// Against rocFFT, packing and bin_scan_kernel, a linear-bin call of the FP32
+// form, the same state (us): 2D 100 56 / 89, 250 59 / 104, 600 72 / 136, 1000
+// 85 / 177; 3D 48 75 / 85, 100 108 / 114, 200 208 / 213, 300 614 / 740, 400
+// 1173 / 1577, 500 2377 / 3093, 640 4192 / 6265, 768 7415 / 10747, 900 15734 /
+// 17175; batches 3D 64 x 48 246 / 266, 32 x 64 234 / 219, 16 x 96 334 / 311;
+// and a context's first call of a side 0.2 to 18 ms against 16 to 300 ms, most
+// of it rocFFT's plan.  A bin's error against extended precision: 2.7e-15 rms at
+// 400^3 (rocFFT 3.2e-15), 1.1e-14 at 48^3 (3.0e-14).
+struct AnyPlan {
+    int L = 0, stages = 0;
+    int rad[12], ns[12];               // radix, product of the earlier radices
+    uint32_t mq[12], mn[12];           // ceil(2^32 / (L / rad)), ceil(2^32 / ns)
+};
+
+// n / d for n < 2^16 from m = ceil(2^32 / d) (d = 1: m wraps to 0)
+__device__ __forceinline__ int fast_div(int n, uint32_t m)
+{
+    return m ? (int)__umulhi((uint32_t)n, m) : n;
+}
+static uint32_t magic_of(uint32_t d) { return (uint32_t)((((uint64_t)1 << 32) + d - 1) / d); }
+
+__device__ __forceinline__ void dft3(double2 (&v)[3])
+{
+    constexpr double h = 0x1.bb67ae8584caap-1;                   // sqrt(3) / 2
+    const double2 t{v[1].x + v[2].x, v[1].y + v[2].y}, d{v[1].x - v[2].x, v[1].y - v[2].y};
+    const double2 m{fma(-0.5, t.x, v[0].x), fma(-0.5, t.y, v[0].y)};
+    v[0] = double2{v[0].x + t.x, v[0].y + t.y};
+    v[1] = double2{fma(h, d.y, m.x), fma(-h, d.x, m.y)};         // m - i h d
+    v[2] = double2{fma(-h, d.y, m.x), fma(h, d.x, m.y)};
+}
+
+__device__ __forceinline__ void dft5(double2 (&v)[5])
+{
+    constexpr double c1 = 0x1.3c6ef372fe950p-2, c2 = -0x1.9e3779b97f4a8p-1;   // cos 2pi/5, 4pi/5
+    constexpr double s1 = 0x1.e6f0e134454ffp-1, s2 = 0x1.2cf2304755a5ep-1;    // sin
+    const double2 a{v[1].x + v[4].x, v[1].y + v[4].y}, b{v[2].x + v[3].x, v[2].y + v[3].y};
+    const double2 d{v[1].x - v[4].x, v[1].y - v[4].y}, e{v[2].x - v[3].x, v[2].y - v[3].y};
+    const double2 p{fma(c1, a.x, fma(c2, b.x, v[0].x)), fma(c1, a.y, fma(c2, b.y, v[0].y))};
+    const double2 q{fma(c2, a.x, fma(c1, b.x, v[0].x)), fma(c2, a.y, fma(c1, b.y, v[0].y))};
+    const double2 r{fma(s1, d.x, s2 * e.x), fma(s1, d.y, s2 * e.y)};
+    const double2 t{fma(s2, d.x, -(s1 * e.x)), fma(s2, d.y, -(s1 * e.y))};
+    v[0] = double2{v[0].x + (a.x + b.x), v[0].y + (a.y + b.y)};
+    v[1] = double2{p.x + r.y, p.y - r.x};                        // p - i r
+    v[4] = double2{p.x - r.y, p.y + r.x};
+    v[2] = double2{q.x + t.y, q.y - t.x};
+    v[3] = double2{q.x - t.y, q.y + t.x};
+}
+
+__device__ __forceinline__ void dft7(double2 (&v)[7])
+{
+    // cos and sin of 2 pi m / 7, m = 1, 2, 3
+    constexpr double c[3] = {0x1.3f3a0e28bedd1p-1, -0x1.c7b90e3024582p-3, -0x1.cd4bca9cb5c71p-1};
+    constexpr double s[3] = {0x1.904c37505de4bp-1, 0x1.f329c0558e969p-1, 0x1.bc4c04d71abc1p-2};
+    double2 a[3], d[3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        a[m] = double2{v[m + 1].x + v[6 - m].x, v[m + 1].y + v[6 - m].y};
+        d[m] = double2{v[m + 1].x - v[6 - m].x, v[m + 1].y - v[6 - m].y};
+    }
+    const double2 z = v[0];
+    v[0] = double2{z.x + (a[0].x + a[1].x + a[2].x), z.y + (a[0].y + a[1].y + a[2].y)};
+#pragma unroll
+    for (int k = 1; k <= 3; ++k) {
+        double2 p = z, r{0.0, 0.0};
+#pragma unroll
+        for (int m = 1; m <= 3; ++m) {
+            const int e = k * m % 7, f = e <= 3 ? e : 7 - e;     // angle 2 pi e / 7
+            const double cc = c[f - 1], ss = e <= 3 ? s[f - 1] : -s[f - 1];
+            p = double2{fma(cc, a[m - 1].x, p.x), fma(cc, a[m - 1].y, p.y)};
+            r = double2{fma(ss, d[m - 1].x, r.x), fma(ss, d[m - 1].y, r.y)};
+        }
+        v[k] = double2{p.x + r.y, p.y - r.x};                    // p - i r
+        v[7 - k] = double2{p.x - r.y, p.y + r.x};
+    }
+}
+
+// 8-point DFT as 2 x 4: DFT4 over the even and the odd points, W_8^k between
+__device__ __forceinline__ void dft8(double2 (&v)[8])
+{
+    constexpr double h = 0x1.6a09e667f3bcdp-1;
+    double2 e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
+    dft4(e);
+    dft4(o);
+    o[1] = double2{h * (o[1].x + o[1].y), h * (o[1].y - o[1].x)};
+    o[2] = double2{o[2].y, -o[2].x};
+    o[3] = double2{h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y)};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        v[k] = double2{e[k].x + o[k].x, e[k].y + o[k].y};
+        v[k + 4] = double2{e[k].x - o[k].x, e[k].y - o[k].y};
+    }
+}
+
+// row stride in LDS of rows of L points (fpad, and the odd extra point)
+__host__ __device__ __forceinline__ int any_ls(int L) { return L + L / 16 + 1; }
+
+// stage t of plan p over rows of p.L points at stride LS: at most
+// PTS = 16 THR points in all
+template <int RAD, int THR>
+__device__ __forceinline__ void any_stage(double2 *buf, const double2 *__restrict__ tw, int ts,
+                                          const AnyPlan &p, int t, int LS, int rows)
+{
+    constexpr int NB = (16 + RAD - 1) / RAD;
+    const int Q = p.L / RAD, Ns = p.ns[t], total = rows * Q;
+    const int tstep = Q / Ns * ts;                       // L / (Ns RAD)
+    double2 v[NB][RAD];
+    int to[NB];                                          // row base and first point written
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+        const int b = threadIdx.x + q * THR;
+        to[q] = -1;
+        if (b < total) {
+            const int row = fast_div(b, p.mq[t]), j = b - row * Q;
+            const int jm = j - fast_div(j, p.mn[t]) * Ns;
+            const double2 *rb = buf + row * LS;
+#pragma unroll
+            for (int k = 0; k < RAD; ++k) v[q][k] = rb[fpad(j + k * Q)];
+            if (Ns > 1) {
+                const int step = jm * tstep;
+#pragma unroll
+                for (int k = 1; k < RAD; ++k) v[q][k] = cmulw(v[q][k], tw[k * step]);
+            }
+            if constexpr (RAD == 16)
+                dft16(v[q]);
+            else if constexpr (RAD == 8)
+                dft8(v[q]);
+            else if constexpr (RAD == 7)
+                dft7(v[q]);
+            else if constexpr (RAD == 5)
+                dft5(v[q]);
+            else if constexpr (RAD == 4)
+                dft4(v[q]);
+            else if constexpr (RAD == 3)
+                dft3(v[q]);
+            else
+                dft2(v[q]);
+            to[q] = (row << 16) | ((j - jm) * RAD + jm);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+        if (to[q] >= 0) {
+            double2 *rb = buf + (to[q] >> 16) * LS;
+            const int o = to[q] & 0xffff;
+#pragma unroll
+            for (int k = 0; k < RAD; ++k) rb[fpad(o + k * Ns)] = v[q][k];
+        }
+    __syncthreads();
+}
+
+// forward DFT of `rows` rows in buf; tw[m ts] = W_L^m
+template <int THR>
+__device__ __forceinline__ void any_rows(double2 *buf, const double2 *__restrict__ tw, int ts,
+                                         const AnyPlan &p, int LS, int rows)
+{
+    for (int t = 0; t < p.stages; ++t) {
+        switch (p.rad[t]) {                              // uniform
+        case 16: any_stage<16, THR>(buf, tw, ts, p, t, LS, rows); break;
+        case 8: any_stage<8, THR>(buf, tw, ts, p, t, LS, rows); break;
+        case 7: any_stage<7, THR>(buf, tw, ts, p, t, LS, rows); break;
+        case 5: any_stage<5, THR>(buf, tw, ts, p, t, LS, rows); break;
+        case 4: any_stage<4, THR>(buf, tw, ts, p, t, LS, rows); break;
+        case 3: any_stage<3, THR>(buf, tw, ts, p, t, LS, rows); break;
+        default: any_stage<2, THR>(buf, tw, ts, p, t, LS, rows); break;
+        }
+    }
+}
+
+// points of a group's rows in LDS, with the rows' padding: R rows of L points,
+// R L <= PTS and R <= kAnyRows, take R (L + L/16 + 1)
+constexpr int kAnyRows = 128;
+template <int PTS>
+constexpr int any_lds() { return PTS + PTS / 16 + kAnyRows; }
+
+struct AnyGeom {
+    int N, R, nrows, GI;               // rows of a group; rows in all; groups of i (Y pass)
+    uint32_t mN, mR;                   // magic_of
+    AnyPlan p;
+};
+
+// Z pass: R rows of N reals per group, as fft_z_kernel
+template <class V>
+__device__ __forceinline__ void any_z_load(double2 *buf, const V *__restrict__ pv, int comp,
+                                           size_t site0, int live, const AnyGeom &g, int LS)
+{
+    using GV = const __attribute__((address_space(1))) V;
+    GV *p = (GV *)pv + site0;
+    // sixteen loads in flight, past the end of the last one again
+    constexpr int U = 16;
+    for (int q0 = 0; q0 < 2 * kFftPts / kFftThr; q0 += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = threadIdx.x + (q0 + u) * kFftThr;
+            const V w = p[e < live ? e : live - 1];
+            v[u] = (double)(comp ? w.y : w.x);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = threadIdx.x + (q0 + u) * kFftThr;
+            const int r = fast_div(e, g.mN), z = e - r * g.N;
+            if (e < live) reinterpret_cast<double *>(buf + r * LS + fpad(z >> 1))[z & 1] = v[u];
+        }
+    }
+}
+
+// the rows' twiddles W_N^m, m < n, read from LDS where TWL (a table of a 3D
+// side fits; a global load in every stage would be waited for)
+template <int THR>
+__device__ __forceinline__ void any_tw(double2 *twl, const double2 *__restrict__ tw, int n, int ts)
+{
+    for (int m = threadIdx.x; m < n; m += THR) twl[m] = tw[m * ts];
+}
+
+template <int ND, bool TWL>
+__global__ void __launch_bounds__(kFftThr)
+any_z_kernel(AnyGeom g, const PkSrc *__restrict__ src, double2 *__restrict__ y,
+             const double2 *__restrict__ tw)
+{
+    __shared__ double2 buf[any_lds<kFftPts>()];
+    __shared__ double2 twl[TWL ? 512 : 1];               // W_M^m
+    if (TWL) any_tw<kFftThr>(twl, tw, g.N / 2, 2);
+    const int N = g.N, M = N / 2, R = g.R, LS = any_ls(M);
+    const uint32_t b = blockIdx.y, row0 = blockIdx.x * (uint32_t)R;
+    const int rows = ((uint32_t)g.nrows - row0 < (uint32_t)R) ? g.nrows - (int)row0 : R;
+    const PkSrc sc = src[b];
+    const size_t site0 = (size_t)row0 * N;
+    if (sc.kind == 0)
+        any_z_load(buf, (const dvec2 *)sc.p, sc.comp, site0, rows * N, g, LS);
+    else if (sc.kind == 1)
+        any_z_load(buf, (const fvec4 *)sc.p, sc.comp, site0, rows * N, g, LS);
+    else
+        any_z_load(buf, (const fvec2 *)sc.p, sc.comp, site0, rows * N, g, LS);
+    __syncthreads();
+    if (TWL)
+        any_rows<kFftThr>(buf, twl, 1, g.p, LS, rows);
+    else
+        any_rows<kFftThr>(buf, tw, 2, g.p, LS, rows);          // W_M^m = W_N^2m
+#pragma unroll 2
+    for (int q = 0; q < kFftPts / kFftThr; ++q) {
+        const int e = threadIdx.x + q * kFftThr;
+        if (e >= R * M) break;
+        const int k = fast_div(e, g.mR), r = e - k * R;
+        if (r >= rows) continue;
+        const double2 a = buf[r * LS + fpad(k)], c = buf[r * LS + fpad(k ? M - k : 0)];
+        const double2 E{0.5 * (a.x + c.x), 0.5 * (a.y - c.y)};
+        const double2 O{0.5 * (a.y + c.y), -0.5 * (a.x - c.x)};
+        const double2 w = cmulw(O, tw[k]);
+        const uint32_t rl = row0 + (uint32_t)r;
+        size_t idx;
+        if (ND == 3) {
+            const uint32_t i = rl / (uint32_t)N, j = rl - i * (uint32_t)N;
+            idx = (((size_t)b * N + i) * M + (uint32_t)k) * N + j;
+        } else {
+            idx = ((size_t)b * M + (uint32_t)k) * N + rl;
+        }
+        y[idx] = double2{E.x + w.x, E.y + w.y};
+    }
+}
+
+// `live` points of rows of N points at stride `pitch` into buf, all of a thread's
+// loads in flight
+template <int PER, int THR>
+__device__ __forceinline__ void any_load(double2 *buf, const double2 *__restrict__ src, int live,
+                                         size_t pitch, const AnyGeom &g, int LS)
+{
+    double vr[PER], vi[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e0 = threadIdx.x + q * THR, e = e0 < live ? e0 : live - 1;
+        const int r = fast_div(e, g.mN);
+        const double2 v = src[(size_t)r * pitch + (e - r * g.N)];
+        vr[q] = v.x;
+        vi[q] = v.y;
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = threadIdx.x + q * THR;
+        const int r = fast_div(e, g.mN);
+        if (e < live) buf[r * LS + fpad(e - r * g.N)] = double2{vr[q], vi[q]};
+    }
+}
+
+// Y pass (3D): rows Y[b][i][k_z][*] of R consecutive i; Y'[b][k_z][k_j][i]
+__global__ void __launch_bounds__(kFftPtsY / 16)
+any_y_kernel(AnyGeom g, const double2 *__restrict__ ya, double2 *__restrict__ yb,
+             const double2 *__restrict__ tw)
+{
+    constexpr int THR = kFftPtsY / 16;
+    __shared__ double2 buf[any_lds<kFftPtsY>()];
+    __shared__ double2 twl[1024];
+    any_tw<THR>(twl, tw, g.N, 1);
+    const int N = g.N, M = N / 2, R = g.R, LS = any_ls(N);
+    const uint32_t ig = blockIdx.x % (uint32_t)g.GI, t = blockIdx.x / (uint32_t)g.GI;
+    const uint32_t kz = t % (uint32_t)M, b = t / (uint32_t)M;
+    const int i0 = (int)ig * R, rows = (N - i0 < R) ? N - i0 : R;
+    const double2 *src = ya + (((size_t)b * N + i0) * M + kz) * N;
+    any_load<kFftPtsY / THR, THR>(buf, src, rows * N, (size_t)M * N, g, LS);
+    __syncthreads();
+    any_rows<THR>(buf, twl, 1, g.p, LS, rows);
+    double2 *dst = yb + ((size_t)b * M + kz) * N * N + i0;
+#pragma unroll 4
+    for (int q = 0; q < kFftPtsY / THR; ++q) {
+        const int e = threadIdx.x + q * THR;
+        if (e < R * N) {
+            const int kj = fast_div(e, g.mR), r = e - kj * R;
+            if (r < rows) dst[(size_t)kj * N + r] = buf[r * LS + fpad(kj)];
+        }
+    }
+}
+
+// last pass with the binning, as fft_bin_kernel; the two halves of a row apart
+// (|k| runs up over the first and down over the second, so each bin present in
+// a chunk of 64 lanes of one half is one run)
+// (LDS: the group's rows, the twiddles, then the bins' sums and tables)
+static size_t any_bin_lds(int N, int R, int waves, int nbins, bool twl)
+{
+    return ((size_t)R * any_ls(N) + (twl ? (size_t)N : 0)) * sizeof(double2) +
+           (size_t)waves * nbins * sizeof(double) + (size_t)nbins * 4 + (size_t)(N / 2) * 2;
+}
+
+template <int ND, int PTS, bool TWL>
+__global__ void __launch_bounds__(PTS / 16)
+any_bin_kernel(AnyGeom g, const double2 *__restrict__ y, const double2 *__restrict__ tw, int nbins,
+               const uint32_t *__restrict__ hi2g, const uint16_t *__restrict__ shellg,
+               KahanP *__restrict__ part)
+{
+    constexpr int THR = PTS / 16, W = THR / 64;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int N = g.N, half = N / 2, R = g.R, LS = any_ls(N);
+    double2 *buf = reinterpret_cast<double2 *>(smem);
+    double2 *twl = buf + R * LS;
+    double *acc = reinterpret_cast<double *>(twl + (TWL ? N : 0));     // [wave][bin]
+    uint32_t *hi2 = reinterpret_cast<uint32_t *>(acc + W * nbins);
+    uint16_t *shell = reinterpret_cast<uint16_t *>(hi2 + nbins);
+    if (TWL) any_tw<THR>(twl, tw, N, 1);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = threadIdx.x; i < nbins; i += THR) {
+        hi2[i] = hi2g[i];
+        for (int w = 0; w < W; ++w) acc[w * nbins + i] = 0.0;
+    }
+    for (int i = threadIdx.x; i < half; i += THR) shell[i] = shellg[i];
+    __syncthreads();
+    double *wacc = acc + wave * nbins;
+    const double2 *yl = y + (size_t)blockIdx.y * g.nrows * N;
+    const uint32_t top = (uint32_t)half * (uint32_t)half;
+    const uint64_t upto = (2ull << lane) - 1;
+    const uint32_t ngroups = ((uint32_t)g.nrows + R - 1) / (uint32_t)R;
+    const uint32_t g0 = (uint32_t)(((uint64_t)ngroups * blockIdx.x) / gridDim.x);
+    const uint32_t g1 = (uint32_t)(((uint64_t)ngroups * (blockIdx.x + 1)) / gridDim.x);
+    // |k|^2 of a row's fixed components
+    auto row_r2 = [&](uint32_t q, bool &zero_plane) -> uint32_t {
+        if (ND == 3) {
+            const uint32_t kz = q / (uint32_t)N, kj = q - kz * (uint32_t)N;
+            const int fj = (int)kj < half ? (int)kj : (int)kj - N;
+            zero_plane = kz == 0;
+            return kz * kz + (uint32_t)(fj * fj);
+        }
+        zero_plane = q == 0;
+        return q * q;
+    };
+    for (uint32_t gq = g0; gq < g1; ++gq) {
+        const uint32_t row0 = gq * (uint32_t)R;
+        const int rows = ((uint32_t)g.nrows - row0 < (uint32_t)R) ? g.nrows - (int)row0 : R;
+        // a group whose rows all lie outside |k| < N/2 is not transformed
+        uint32_t rmin = 0xffffffffu;
+        bool zp;
+        for (int r = 0; r < rows; ++r) {
+            const uint32_t r2 = row_r2(row0 + (uint32_t)r, zp);
+            rmin = r2 < rmin ? r2 : rmin;
+        }
+        if (rmin >= top) continue;
+        any_load<PTS / THR, THR>(buf, yl + (size_t)row0 * N, rows * N, (size_t)N, g, LS);
+        __syncthreads();
+        if (TWL)
+            any_rows<THR>(buf, twl, 1, g.p, LS, rows);
+        else
+            any_rows<THR>(buf, tw, 1, g.p, LS, rows);
+        for (int r = wave; r < rows; r += W) {
+            const uint32_t r2 = row_r2(row0 + (uint32_t)r, zp);
+            if (r2 >= top) continue;                 // the whole row has |k| >= N/2
+            for (int h = 0; h < 2; ++h) {
+                const int x1 = h ? N : half;
+                for (int x0 = h ? half : 0; x0 < x1; x0 += 64) {
+                    // the smallest |f| of the chunk decides whether any lane is inside
+                    const int last = x0 + 63 < x1 ? x0 + 63 : x1 - 1;
+                    const int fmin = h ? N - last : x0;
+                    if (r2 + (uint32_t)(fmin * fmin) >= top) continue;
+                    const int x = x0 + lane;
+                    const int fx = h ? x - N : x;
+                    const uint32_t k2 = r2 + (uint32_t)(fx * fx);
+                    const bool on = x < x1 && k2 < top && k2 > 0;
+                    int b;
+                    double v = 0.0;
+                    if (on) {
+                        uint32_t sh = (uint32_t)__builtin_amdgcn_sqrtf((float)k2);
+                        if (sh * sh > k2) --sh;
+                        if ((sh + 1) * (sh + 1) <= k2) ++sh;
+                        b = shell[sh];
+                        while (hi2[b] <= k2) ++b;
+                        const double2 f = buf[r * LS + fpad(x)];
+                        const double p2 = f.x * f.x + f.y * f.y;
+                        v = zp ? p2 : 2.0 * p2;
+                    } else {
+                        b = (k2 == 0) ? -1 : nbins;
+                    }
+                    const int bprev = __builtin_amdgcn_update_dpp(-2, b, 0x138, 0xf, 0xf, false);
+                    const uint64_t heads = __ballot(bprev != b);
+                    const int start = 63 - __clzll(heads & upto);
+                    const int len = lane - start;
+                    double u;
+                    u = dpp_take<0x111, 0xf>(v);
+                    if (len >= 1) v += u;
+                    u = dpp_take<0x112, 0xf>(v);
+                    if (len >= 2) v += u;
+                    u = dpp_take<0x114, 0xf>(v);
+                    if (len >= 4) v += u;
+                    u = dpp_take<0x118, 0xf>(v);
+                    if (len >= 8) v += u;
+                    u = dpp_take<0x142, 0xa>(v);
+                    if (len > (lane & 15)) v += u;
+                    u = dpp_take<0x143, 0xc>(v);
+                    if (len > (lane & 31)) v += u;
+                    const bool fin = lane == 63 || (((heads >> lane) >> 1) & 1ull);
+                    if (fin && b >= 0 && b < nbins) wacc[b] += v;
+                }
+            }
+        }
+        __syncthreads();                             // before the next group's loads
+    }
+    for (int i = threadIdx.x; i < nbins; i += THR) {
+        KahanP a{acc[i], 0.0};
+        for (int w = 1; w < W; ++w) a = kmergep(a, KahanP{acc[w * nbins + i], 0.0});
+        part[((size_t)blockIdx.y * nbins + i) * gridDim.x + blockIdx.x] = a;
+    }
+}
+
+// stages of a row of L points; false if L has a prime factor above 7
+static bool any_plan(int L, AnyPlan &p)
+{
+    p.L = L;
+    p.stages = 0;
+    int n = L, ns = 1;
+    for (int r : {16, 8, 4, 2, 7, 5, 3})
+        while (n % r == 0 && p.stages < 12) {
+            p.rad[p.stages] = r;
+            p.ns[p.stages] = ns;
+            p.mq[p.stages] = magic_of((uint32_t)(L / r));
+            p.mn[p.stages] = magic_of((uint32_t)ns);
+            ns *= r;
+            n /= r;
+            ++p.stages;
+        }
+    return n == 1;
+}
+
 // bins of a lattice of side N as ranges [lo, hi) of the integer |k|^2, and
 // the work items (bounding-box rows in chunks of kPkRows) of each bin
 struct BinLayout {
@@ -1254,6 +1727,94 @@ static int pk_raw_own(Context *c, const PkSrc *srcs, int n, int N, const BinLayo
     return bin_finish(c, n, B, t, nblk, g, hpk, hks, hcnt);
 }
 
+// rows of a group: what the LDS takes, and few enough that a small lattice's
+// rows reach every CU
+static int any_group(const Context *c, int most, int nrows, int n)
+{
+    const int64_t cu = std::max(1, c->num_cu);
+    const int64_t spread = ((int64_t)nrows * n + cu - 1) / cu;
+    return (int)std::min<int64_t>(std::min(most, kAnyRows), std::min<int64_t>(spread, nrows));
+}
+
+// points and rows of the last pass's groups for rows of N points (the order of the
+// bins' sums, so the same for one spectrum and a batch), and the LDS it may take; the twiddles go to LDS where a group's rows leave room
+static int any_bin_pts(int N) { return N > 2048 ? 4096 : 2048; }
+static int any_bin_rows(const Context *c, int N)
+{
+    const int nrows = (c->nd == 3) ? N / 2 * N : N / 2;
+    return std::min(nrows, std::max(any_group(c, any_bin_pts(N) / N, nrows, 1),
+                                    std::min(512 / N, kAnyRows)));
+}
+constexpr size_t kAnyBinLds = 64 * 1024;
+
+// Sides the run-time transform takes: those whose rows, their bins' sums and
+// tables fit the last pass's LDS (2D linear bins to N of about 2000)
+static bool any_fft_ok(const Context *c, int N, const BinLayout &B)
+{
+    if (c->pk_rocfft || N < 16 || N > (c->nd == 3 ? 1024 : 4096) || !B.scan) return false;
+    AnyPlan p;
+    if (!any_plan(N, p) || !any_plan(N / 2, p)) return false;
+    const int pts = any_bin_pts(N);
+    return any_bin_lds(N, any_bin_rows(c, N), pts / 16 / 64, B.nbins, false) <= kAnyBinLds;
+}
+
+// The n spectra of side N by the run-time transform (any_fft_ok).
+static int pk_raw_any(Context *c, const PkSrc *srcs, int n, int N, const BinLayout &B,
+                      std::vector<double> &hpk, std::vector<double> &hks,
+                      std::vector<long long> &hcnt)
+{
+    FftPlan *p = nullptr;
+    AXS_TRY(get_own(c, N, n, &p));
+    const int M = N / 2, pts = any_bin_pts(N);
+    AnyGeom z{}, y{}, x{};
+    z.N = y.N = x.N = N;
+    z.mN = y.mN = x.mN = magic_of((uint32_t)N);
+    any_plan(M, z.p);
+    any_plan(N, y.p);
+    any_plan(N, x.p);
+    z.nrows = (c->nd == 3) ? N * N : N;
+    z.R = any_group(c, kFftPts / M, z.nrows, n);
+    y.R = any_group(c, kFftPtsY / N, N, n * M);
+    y.GI = (N + y.R - 1) / y.R;
+    y.R = (N + y.GI - 1) / y.GI;                    // groups of equal size
+    x.nrows = (c->nd == 3) ? M * N : M;
+    x.R = any_bin_rows(c, N);
+    z.mR = magic_of((uint32_t)z.R);
+    y.mR = magic_of((uint32_t)y.R);
+    const uint32_t groups = ((uint32_t)x.nrows + x.R - 1) / (uint32_t)x.R;
+    const uint32_t nblk = std::max<uint32_t>(1, std::min<uint32_t>(groups, 4096));
+    ScanTabs t;
+    AXS_TRY(scan_tabs(c, B, n, nblk, t));
+    Context::PkGeom *g = nullptr;
+    AXS_TRY(bin_geometry(c, B, t, &g));
+    AXS_HIP_TRY(hipMemcpyAsync(t.src, srcs, (size_t)n * sizeof(PkSrc), hipMemcpyHostToDevice,
+                               c->stream));
+    const unsigned gz = (unsigned)((z.nrows + z.R - 1) / z.R);
+    const double2 *last = p->ya;
+    if (c->nd == 3) {
+        hipLaunchKernelGGL((any_z_kernel<3, true>), dim3(gz, (unsigned)n), dim3(kFftThr), 0,
+                           c->stream, z, t.src, p->ya, p->tw);
+        hipLaunchKernelGGL(any_y_kernel, dim3((unsigned)n * M * y.GI), dim3(kFftPtsY / 16), 0,
+                           c->stream, y, p->ya, p->yb, p->tw);
+        last = p->yb;
+    } else {
+        auto kz = (M <= 512) ? any_z_kernel<2, true> : any_z_kernel<2, false>;
+        hipLaunchKernelGGL(kz, dim3(gz, (unsigned)n), dim3(kFftThr), 0, c->stream, z, t.src,
+                           p->ya, p->tw);
+    }
+    const int waves = pts / 16 / 64;
+    const bool twl = any_bin_lds(N, x.R, waves, B.nbins, true) <= kAnyBinLds;
+    const size_t lds = any_bin_lds(N, x.R, waves, B.nbins, twl);
+    auto kb = (c->nd == 3) ? (twl ? any_bin_kernel<3, 2048, true> : any_bin_kernel<3, 2048, false>)
+              : (pts == 4096) ? any_bin_kernel<2, 4096, false>
+              : twl           ? any_bin_kernel<2, 2048, true>
+                              : any_bin_kernel<2, 2048, false>;
+    hipLaunchKernelGGL(kb, dim3(nblk, (unsigned)n), dim3(pts / 16), lds, c->stream, x, last, p->tw,
+                       B.nbins, t.hi, t.shell, t.part);
+    AXS_HIP_TRY(hipGetLastError());
+    return bin_finish(c, n, B, t, nblk, g, hpk, hks, hcnt);
+}
+
 // Raw bin sums (|F|^2, |k| and mode counts per bin, before the
 // normalisation) of n real fields of side N in one batched transform:
 // source q's bins go to hpk / hks / hcnt + q nbins.
@@ -1263,6 +1824,7 @@ static int pk_raw(Context *c, const PkSrc *srcs, int n, int N, const BinLayout &
 {
     const int nbins = B.nbins;
     if (own_fft_ok(c, N, B)) return pk_raw_own(c, srcs, n, N, B, hpk, hks, hcnt);
+    if (any_fft_ok(c, N, B)) return pk_raw_any(c, srcs, n, N, B, hpk, hks, hcnt);
     FftPlan *plan = nullptr;
     AXS_TRY(get_plan(c, N, n, &plan));
     const uint32_t L = (uint32_t)((c->nd == 3) ? (int64_t)N * N * N : (int64_t)N * N);

@@ -274,8 +274,8 @@ def ensemble_leg(np, axs, name, T0, steps_override=0, autotune=True):
             log(f"[bench] {name} {prec}: {len(Ns)} members, tuned {cfg} ({tuned_ms:.3f} ms)")
         else:
             cfg = lat.kernel_config()
-        # the sampling path's one-time set-up (rocFFT builds and plans its
-        # kernels for each side on first use): one sample of the initial
+        # the sampling path's one-time set-up (the spectra's buffers and
+        # transform of each side on first use): one sample of the initial
         # state, timed on its own
         t0 = time.perf_counter()
         lat.string_counts()

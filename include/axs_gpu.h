@@ -209,7 +209,7 @@ int axs_member_energy_noalloc(axs_ctx *ctx, int member, double out[3]);
  * member `member`: AXS_BIN_LINEAR gives the reference's N/2 unit-width bins
  * (nbins ignored; arrays need N/2 entries); AXS_BIN_LOG gives nbins log bins
  * with pk the mean |F|^2 per mode.  ks, pk, count: one entry per bin.  Empty
- * bins have count 0.  Transform by rocFFT, bins in compensated FP64.       */
+ * bins have count 0.  FP64 transform, bins in compensated FP64.            */
 int axs_member_powerspec(axs_ctx *ctx, int member, int binning, int nbins,
                          double *ks, double *pk, int32_t *count);
 int axs_powerspec(axs_ctx *ctx, int binning, int nbins,
@@ -233,7 +233,7 @@ int axs_member_powerspec_field(axs_ctx *ctx, int member, int field, int binning,
 
 /* The spectra of every member in one call (ensembles have no reference
  * counterpart; each member's spectrum is the axs_member_powerspec one).
- * Members of one side share batched rocFFT transforms and one binning
+ * Members of one side share batched transforms and one binning
  * launch, with one synchronisation per batch.  Member r's bins start at
  * entry sum_{q<r} nb_q of ks, pk and count, nb_q = N_q/2 (AXS_BIN_LINEAR)
  * or nbins (AXS_BIN_LOG).                                                  */
