@@ -507,9 +507,8 @@ fold_rows_kernel(int nbins, uint32_t nblk, const KahanP *__restrict__ part,
 //   Y  rows along j: N-point DFTs, written as Y'[k_z][k_j][i].
 //   X  rows along i: N-point DFTs, then every mode's w |F|^2 (w = 1 at
 //      k_z = 0, else 2 for the Hermitian partner) binned as bin_scan_kernel
-//      does; along a row |k| runs up over the first half and down over the
-//      second, so the 64 lanes of a chunk (N >= 128) still hold each bin
-//      present as one run.
+//      does, the modes fx and -fx of a row added first: over fx = 0 .. N/2 - 1
+//      |k| grows, so the 64 lanes of a chunk hold each bin present as one run.
 // 2D (f[j][i]) is Z along i, written as Y[k][j], then the binning pass
 // along j.  A work-group transforms kFftPts complex points in LDS, rows of
 // one length L: radix-4 Stockham stages (one radix-2 stage first when
@@ -795,6 +794,104 @@ fft_y_kernel(const double2 *__restrict__ ya, double2 *__restrict__ yb,
     }
 }
 
+// C chunks of 64 frequencies fx = f0 + 64 c + lane of one transformed row, its
+// modes fx and -fx summed first (one |k|, one bin): C segmented scans side by side,
+// then the runs' sums into the wave's accumulators, chunk by chunk.  The scan's
+// chain of dependent lane moves is what a wave waits for (one or two waves a SIMD):
+// half the chunks and two chains at once took a linear-bin call from 12.7 to 11.5
+// ms at 1024^3, 1535 to 1431 us at 512^3, 1174 to 1085 at 400^3, 4191 to 3900 at
+// 640^3 and a batch of 32 x 64^3 from 253 to 235; four chains at once no further.
+template <int C>
+__device__ __forceinline__ void bin_chunks(const double2 *rb, int N, int half, int f0, int lane,
+                                           uint64_t upto, uint32_t r2, uint32_t top, double w,
+                                           int nbins, const uint16_t *shell, const uint32_t *hi2,
+                                           double *wacc)
+{
+    int b[C];
+    uint32_t k2[C], hi[C];
+    bool on[C];
+    double v[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int f = f0 + 64 * c + lane;
+        k2[c] = r2 + (uint32_t)(f * f);
+        on[c] = f < half && k2[c] < top && k2[c] > 0;
+        uint32_t sh = (uint32_t)__builtin_amdgcn_sqrtf((float)k2[c]);
+        if (sh * sh > k2[c]) --sh;
+        if ((sh + 1) * (sh + 1) <= k2[c]) ++sh;
+        b[c] = on[c] ? (int)shell[sh] : 0;
+        const int x = on[c] ? f : 0;
+        const double2 p = rb[fpad(x)], q = rb[fpad(x ? N - x : 0)];
+        const double p2 = p.x * p.x + p.y * p.y, q2 = q.x * q.x + q.y * q.y;
+        v[c] = on[c] ? w * (x ? p2 + q2 : p2) : 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) hi[c] = hi2[b[c]];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        if (on[c])
+            while (hi[c] <= k2[c]) hi[c] = hi2[++b[c]];
+        else
+            b[c] = (k2[c] == 0) ? -1 : nbins;
+    }
+    int len[C];
+    bool last[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int bprev = __builtin_amdgcn_update_dpp(-2, b[c], 0x138, 0xf, 0xf, false);
+        const uint64_t heads = __ballot(bprev != b[c]);
+        len[c] = lane - (63 - __clzll(heads & upto));
+        last[c] = lane == 63 || (((heads >> lane) >> 1) & 1ull);
+    }
+    double u[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = dpp_take<0x111, 0xf>(v[c]);
+        if (len[c] >= 1) v[c] += u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = dpp_take<0x112, 0xf>(v[c]);
+        if (len[c] >= 2) v[c] += u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = dpp_take<0x114, 0xf>(v[c]);
+        if (len[c] >= 4) v[c] += u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = dpp_take<0x118, 0xf>(v[c]);
+        if (len[c] >= 8) v[c] += u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = dpp_take<0x142, 0xa>(v[c]);
+        if (len[c] > (lane & 15)) v[c] += u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        u[c] = dpp_take<0x143, 0xc>(v[c]);
+        if (len[c] > (lane & 31)) v[c] += u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+        if (last[c] && b[c] >= 0 && b[c] < nbins) wacc[b[c]] += v[c];
+}
+
+// the modes of one transformed row, r2 = |k|^2 of its fixed components: two
+// chunks at a time while both hold a mode inside |k| < N/2
+__device__ __forceinline__ void bin_row(const double2 *rb, int N, int half, int lane, uint64_t upto,
+                                        uint32_t r2, uint32_t top, double w, int nbins,
+                                        const uint16_t *shell, const uint32_t *hi2, double *wacc)
+{
+    int f0 = 0;
+    for (; f0 + 64 < half && r2 + (uint32_t)((f0 + 64) * (f0 + 64)) < top; f0 += 128)
+        bin_chunks<2>(rb, N, half, f0, lane, upto, r2, top, w, nbins, shell, hi2, wacc);
+    if (f0 < half && r2 + (uint32_t)(f0 * f0) < top)
+        bin_chunks<1>(rb, N, half, f0, lane, upto, r2, top, w, nbins, shell, hi2, wacc);
+}
+
 // Last pass with the binning: rows along the last axis (3D: Y'[b][k_z][k_j]
 // [*] along i; 2D: Y[b][k][*] along j), R = kFftPts / N rows per group; each
 // work-group takes a contiguous run of groups (blockIdx.y = lattice); each
@@ -879,49 +976,8 @@ fft_bin_kernel(const double2 *__restrict__ y, const double2 *__restrict__ tw, in
                 zero_plane = g == 0;
             }
             if (r2 >= top) continue;                 // the whole row has |k| >= N/2
-            for (int x0 = 0; x0 < N; x0 += 64) {
-                // chunks lie in one half of the row (N >= 128): the smallest
-                // |f| of the chunk decides whether any lane is inside
-                const int fmin = x0 < half ? x0 : N - (x0 + 63);
-                if (r2 + (uint32_t)(fmin * fmin) >= top) continue;
-                const int x = x0 + lane;
-                const int fx = x < half ? x : x - N;
-                const uint32_t k2 = r2 + (uint32_t)(fx * fx);
-                const bool on = k2 < top && k2 > 0;
-                int b;
-                double v = 0.0;
-                if (on) {
-                    uint32_t sh = (uint32_t)__builtin_amdgcn_sqrtf((float)k2);
-                    if (sh * sh > k2) --sh;
-                    if ((sh + 1) * (sh + 1) <= k2) ++sh;
-                    b = shell[sh];
-                    while (hi2[b] <= k2) ++b;
-                    const double2 f = buf[r * LS + fpad(x)];
-                    const double p2 = f.x * f.x + f.y * f.y;
-                    v = zero_plane ? p2 : 2.0 * p2;
-                } else {
-                    b = (k2 == 0) ? -1 : nbins;
-                }
-                const int bprev = __builtin_amdgcn_update_dpp(-2, b, 0x138, 0xf, 0xf, false);
-                const uint64_t heads = __ballot(bprev != b);
-                const int start = 63 - __clzll(heads & upto);
-                const int len = lane - start;
-                double u;
-                u = dpp_take<0x111, 0xf>(v);
-                if (len >= 1) v += u;
-                u = dpp_take<0x112, 0xf>(v);
-                if (len >= 2) v += u;
-                u = dpp_take<0x114, 0xf>(v);
-                if (len >= 4) v += u;
-                u = dpp_take<0x118, 0xf>(v);
-                if (len >= 8) v += u;
-                u = dpp_take<0x142, 0xa>(v);
-                if (len > (lane & 15)) v += u;
-                u = dpp_take<0x143, 0xc>(v);
-                if (len > (lane & 31)) v += u;
-                const bool last = lane == 63 || (((heads >> lane) >> 1) & 1ull);
-                if (last && b >= 0 && b < nbins) wacc[b] += v;
-            }
+            bin_row(buf + r * LS, N, half, lane, upto, r2, top, zero_plane ? 1.0 : 2.0, nbins, shell,
+                    hi2, wacc);
         }
         __syncthreads();                             // before the next group's loads
     }
@@ -944,17 +1000,18 @@ fft_bin_kernel(const double2 *__restrict__ y, const double2 *__restrict__ tw, in
 // the three passes' 3 GB would take 0.6 ms.  So a thread's loads are in flight
 // together (clamped to the last row, not guarded) and the twiddles lie in LDS
 // (any_tw), the two together 1634 -> 1173 us at 400^3; and a small lattice's rows
-// are spread over all CUs (any_group: 113 -> 75 us at 48^3).  Radices 6, 10, 12, 14 and 15 as two coprime factors, which save
-// a stage of three or four at some sides, gained 7 to 14 % at 300^3, 500^3 and
+// are spread over all CUs (any_group: 113 -> 75 us at 48^3).  Radices 6, 10, 12,
+// 14 and 15 as two coprime factors, which save a stage of three or four at some
+// sides, gained 7 to 14 % at 300^3, 500^3 and
 // 900^3, nothing at 200^3, 320^3 and 400^3, and lost 3 % at 640^3: not taken.
 // Against rocFFT, packing and bin_scan_kernel, a linear-bin call of the FP32
-// form, the same state (us): 2D 100 56 / 89, 250 59 / 104, 600 72 / 136, 1000
-// 85 / 177; 3D 48 75 / 85, 100 108 / 114, 200 208 / 213, 300 614 / 740, 400
-// 1173 / 1577, 500 2377 / 3093, 640 4192 / 6265, 768 7415 / 10747, 900 15734 /
-// 17175; batches 3D 64 x 48 246 / 266, 32 x 64 234 / 219, 16 x 96 334 / 311;
-// and a context's first call of a side 0.2 to 18 ms against 16 to 300 ms, most
-// of it rocFFT's plan.  A bin's error against extended precision: 2.7e-15 rms at
-// 400^3 (rocFFT 3.2e-15), 1.1e-14 at 48^3 (3.0e-14).
+// form, the same state (us): 2D 100 54 / 96, 250 57 / 102, 600 68 / 141, 1000
+// 85 / 186; 3D 48 81 / 95, 100 106 / 117, 200 205 / 209, 300 597 / 749, 400
+// 1083 / 1572, 500 2262 / 3093, 640 3916 / 6273, 768 7295 / 10354, 900 15097 /
+// 17206; batches 3D 64 x 48 252 / 291, 32 x 64 231 / 233, 16 x 96 327 / 323, but
+// 256 x 16 239 / 213; and a context's first call of a side 0.2 to 17 ms against 16
+// to 300 ms, most of it rocFFT's plan.  A bin's error against extended precision:
+// 2.7e-15 rms at 400^3 (rocFFT 3.2e-15), 1.1e-14 at 48^3 (3.0e-14).
 struct AnyPlan {
     int L = 0, stages = 0;
     int rad[12], ns[12];               // radix, product of the earlier radices
@@ -1259,9 +1316,7 @@ any_y_kernel(AnyGeom g, const double2 *__restrict__ ya, double2 *__restrict__ yb
     }
 }
 
-// last pass with the binning, as fft_bin_kernel; the two halves of a row apart
-// (|k| runs up over the first and down over the second, so each bin present in
-// a chunk of 64 lanes of one half is one run)
+// last pass with the binning, as fft_bin_kernel
 // (LDS: the group's rows, the twiddles, then the bins' sums and tables)
 static size_t any_bin_lds(int N, int R, int waves, int nbins, bool twl)
 {
@@ -1330,52 +1385,8 @@ any_bin_kernel(AnyGeom g, const double2 *__restrict__ y, const double2 *__restri
         for (int r = wave; r < rows; r += W) {
             const uint32_t r2 = row_r2(row0 + (uint32_t)r, zp);
             if (r2 >= top) continue;                 // the whole row has |k| >= N/2
-            for (int h = 0; h < 2; ++h) {
-                const int x1 = h ? N : half;
-                for (int x0 = h ? half : 0; x0 < x1; x0 += 64) {
-                    // the smallest |f| of the chunk decides whether any lane is inside
-                    const int last = x0 + 63 < x1 ? x0 + 63 : x1 - 1;
-                    const int fmin = h ? N - last : x0;
-                    if (r2 + (uint32_t)(fmin * fmin) >= top) continue;
-                    const int x = x0 + lane;
-                    const int fx = h ? x - N : x;
-                    const uint32_t k2 = r2 + (uint32_t)(fx * fx);
-                    const bool on = x < x1 && k2 < top && k2 > 0;
-                    int b;
-                    double v = 0.0;
-                    if (on) {
-                        uint32_t sh = (uint32_t)__builtin_amdgcn_sqrtf((float)k2);
-                        if (sh * sh > k2) --sh;
-                        if ((sh + 1) * (sh + 1) <= k2) ++sh;
-                        b = shell[sh];
-                        while (hi2[b] <= k2) ++b;
-                        const double2 f = buf[r * LS + fpad(x)];
-                        const double p2 = f.x * f.x + f.y * f.y;
-                        v = zp ? p2 : 2.0 * p2;
-                    } else {
-                        b = (k2 == 0) ? -1 : nbins;
-                    }
-                    const int bprev = __builtin_amdgcn_update_dpp(-2, b, 0x138, 0xf, 0xf, false);
-                    const uint64_t heads = __ballot(bprev != b);
-                    const int start = 63 - __clzll(heads & upto);
-                    const int len = lane - start;
-                    double u;
-                    u = dpp_take<0x111, 0xf>(v);
-                    if (len >= 1) v += u;
-                    u = dpp_take<0x112, 0xf>(v);
-                    if (len >= 2) v += u;
-                    u = dpp_take<0x114, 0xf>(v);
-                    if (len >= 4) v += u;
-                    u = dpp_take<0x118, 0xf>(v);
-                    if (len >= 8) v += u;
-                    u = dpp_take<0x142, 0xa>(v);
-                    if (len > (lane & 15)) v += u;
-                    u = dpp_take<0x143, 0xc>(v);
-                    if (len > (lane & 31)) v += u;
-                    const bool fin = lane == 63 || (((heads >> lane) >> 1) & 1ull);
-                    if (fin && b >= 0 && b < nbins) wacc[b] += v;
-                }
-            }
+            bin_row(buf + r * LS, N, half, lane, upto, r2, top, zp ? 1.0 : 2.0, nbins, shell, hi2,
+                    wacc);
         }
         __syncthreads();                             // before the next group's loads
     }
