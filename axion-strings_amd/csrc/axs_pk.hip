@@ -1243,25 +1243,36 @@ any_z_kernel(AnyGeom g, const PkSrc *__restrict__ src, double2 *__restrict__ y,
         any_rows<kFftThr>(buf, twl, 1, g.p, LS, rows);
     else
         any_rows<kFftThr>(buf, tw, 2, g.p, LS, rows);          // W_M^m = W_N^2m
-#pragma unroll 2
-    for (int q = 0; q < kFftPts / kFftThr; ++q) {
-        const int e = threadIdx.x + q * kFftThr;
-        if (e >= R * M) break;
-        const int k = fast_div(e, g.mR), r = e - k * R;
-        if (r >= rows) continue;
-        const double2 a = buf[r * LS + fpad(k)], c = buf[r * LS + fpad(k ? M - k : 0)];
-        const double2 E{0.5 * (a.x + c.x), 0.5 * (a.y - c.y)};
-        const double2 O{0.5 * (a.y + c.y), -0.5 * (a.x - c.x)};
-        const double2 w = cmulw(O, tw[k]);
-        const uint32_t rl = row0 + (uint32_t)r;
-        size_t idx;
-        if (ND == 3) {
-            const uint32_t i = rl / (uint32_t)N, j = rl - i * (uint32_t)N;
-            idx = (((size_t)b * N + i) * M + (uint32_t)k) * N + j;
-        } else {
-            idx = ((size_t)b * M + (uint32_t)k) * N + rl;
+    // the table's loads of eight points in flight, past the end of the last again
+    constexpr int U = 8;
+    for (int q0 = 0; q0 < kFftPts / kFftThr; q0 += U) {
+        double wr[U], wi[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e0 = threadIdx.x + (q0 + u) * kFftThr, e = e0 < R * M ? e0 : R * M - 1;
+            const double2 w = tw[fast_div(e, g.mR)];
+            wr[u] = w.x;
+            wi[u] = w.y;
         }
-        y[idx] = double2{E.x + w.x, E.y + w.y};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = threadIdx.x + (q0 + u) * kFftThr;
+            const int k = fast_div(e, g.mR), r = e - k * R;
+            if (e >= R * M || r >= rows) continue;
+            const double2 a = buf[r * LS + fpad(k)], c = buf[r * LS + fpad(k ? M - k : 0)];
+            const double2 E{0.5 * (a.x + c.x), 0.5 * (a.y - c.y)};
+            const double2 O{0.5 * (a.y + c.y), -0.5 * (a.x - c.x)};
+            const double2 w = cmulw(O, double2{wr[u], wi[u]});
+            const uint32_t rl = row0 + (uint32_t)r;
+            size_t idx;
+            if (ND == 3) {
+                const uint32_t i = rl / (uint32_t)N, j = rl - i * (uint32_t)N;
+                idx = (((size_t)b * N + i) * M + (uint32_t)k) * N + j;
+            } else {
+                idx = ((size_t)b * M + (uint32_t)k) * N + rl;
+            }
+            y[idx] = double2{E.x + w.x, E.y + w.y};
+        }
     }
 }
 
