@@ -1007,7 +1007,7 @@ fft_bin_kernel(const double2 *__restrict__ y, const double2 *__restrict__ tw, in
 // Against rocFFT, packing and bin_scan_kernel, a linear-bin call of the FP32
 // form, the same state (us): 2D 100 54 / 96, 250 57 / 102, 600 68 / 141, 1000
 // 85 / 186; 3D 48 81 / 95, 100 106 / 117, 200 205 / 209, 300 597 / 749, 400
-// 1083 / 1572, 500 2262 / 3093, 640 3916 / 6273, 768 7295 / 10354, 900 15097 /
+// 1083 / 1572, 500 2262 / 3093, 640 3850 / 6273, 768 7295 / 10354, 900 15097 /
 // 17206; batches 3D 64 x 48 252 / 291, 32 x 64 231 / 233, 16 x 96 327 / 323, but
 // 256 x 16 239 / 213; and a context's first call of a side 0.2 to 17 ms against 16
 // to 300 ms, most of it rocFFT's plan.  A bin's error against extended precision:
@@ -1244,6 +1244,7 @@ any_z_kernel(AnyGeom g, const PkSrc *__restrict__ src, double2 *__restrict__ y,
     else
         any_rows<kFftThr>(buf, tw, 2, g.p, LS, rows);          // W_M^m = W_N^2m
     // the table's loads of eight points in flight, past the end of the last again
+    // (a whole call at 640^3 3924 -> 3850 us; small sides unchanged)
     constexpr int U = 8;
     for (int q0 = 0; q0 < kFftPts / kFftThr; q0 += U) {
         double wr[U], wi[U];
