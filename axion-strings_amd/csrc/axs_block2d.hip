@@ -224,7 +224,7 @@ int block2d_depth(const Context *c)
         if (sites > most) return 0;
     }
     // the grid: one group per block
-    if (block2d_tiles(c, block2d_rows(c)) > (uint64_t)INT32_MAX) return 0;
+    if (block2d_tiles(c, block2d_rows(c)) * kBlkItems > kMaxGridItems) return 0;
     return blk_depth(RAD);
 }
 

@@ -19,6 +19,7 @@
 #include "axs_internal.hpp"
 #include "axs_lattice.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace axs {
@@ -167,7 +168,7 @@ block3d_batch_kernel(const BatchMember *__restrict__ mem, int n_members, int d,
 
 // Runs where the marching kernels do not (a member with a side below 64), with
 // the 7-point stencil; in FP64 up to 1024 cubes, about where the one-step
-// kernel catches up.  Measured in us a step, cubes / one-step kernel: FP64 16^3
+// kernel catches up; in FP32 up to the launch limit of 2^22 cubes.  In us a step, cubes / one-step kernel: FP64 16^3
 // 2.9 / 3.5, 48^3 4.1 / 8.1, 62^3 (512 cubes) 6.8 / 10.1, forty of 32^3 (2560)
 // 37.5 / 33.1; FP32 16^3 1.7 / 2.6, 62^3 3.0 / 6.0, forty of 32^3 11.0 / 13.1.
 // Wider stencils gain at most 1.2x (radius 2, 62^3) and lose up to 2x: not built.
@@ -183,7 +184,9 @@ int block3d_depth(const Context *c)
         const uint64_t t = (uint64_t)((m.N + kCubeOut - 1) / kCubeOut);
         cubes += t * t * t;
     }
-    const uint64_t most = (c->prec == AXS_FP64) ? 4 * (uint64_t)c->num_cu : (uint64_t)INT32_MAX;
+    const uint64_t grid = kMaxGridItems / kCubeItems;
+    const uint64_t most = (c->prec == AXS_FP64) ? std::min<uint64_t>(4 * (uint64_t)c->num_cu, grid)
+                                                : grid;
     return (small && cubes <= most) ? kCubeDepth : 0;
 }
 

@@ -335,6 +335,9 @@ int prepare_march2d_items(Context *c, int D);
 int launch_march2d(Context *c, int src, const StepScalars *s, int depth);
 // higher-order stencils (radius 2-4), 2D (axs_march2d_hi.hip)
 int launch_march2d_high_order(Context *c, int src, const StepScalars *s, int depth, bool pf);
+// work-items of one launch along x: a grid's groups times their size has to
+// stay below 2^32
+constexpr uint64_t kMaxGridItems = ((uint64_t)1 << 32) - 1;
 // small lattices (axs_block2d.hip, axs_block3d.hip): most steps of one pass, or
 // 0 where the strip and marching kernels run; d <= block_depth steps in one pass
 int block_depth(const Context *c);
