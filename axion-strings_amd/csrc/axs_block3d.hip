@@ -19,7 +19,6 @@
 #include "axs_internal.hpp"
 #include "axs_lattice.hpp"
 
-#include <algorithm>
 #include <type_traits>
 
 namespace axs {
@@ -167,10 +166,17 @@ block3d_batch_kernel(const BatchMember *__restrict__ mem, int n_members, int d,
 }
 
 // Runs where the marching kernels do not (a member with a side below 64), with
-// the 7-point stencil; in FP64 up to 1024 cubes, about where the one-step
-// kernel catches up; in FP32 up to the launch limit of 2^22 cubes.  In us a step, cubes / one-step kernel: FP64 16^3
-// 2.9 / 3.5, 48^3 4.1 / 8.1, 62^3 (512 cubes) 6.8 / 10.1, forty of 32^3 (2560)
-// 37.5 / 33.1; FP32 16^3 1.7 / 2.6, 62^3 3.0 / 6.0, forty of 32^3 11.0 / 13.1.
+// the 7-point stencil, up to the launch limit (2^22 cubes).  In FP64 one group
+// is resident per CU, so a pass takes as long as its rounds of one cube per CU,
+// 4.1 us a step each, against about 6 us and 22 ps a site for the one-step
+// kernel: the cubes run while that is less, and for four rounds at most (as far
+// as was measured).  In us a step, cubes / one-step kernel: 48^3 4.2 / 8.2, two
+// of 48^3 8.2 / 8.8, four (864 cubes) 16.1 / 15.6, 62^3 7.0 / 9.9, two 14.2 / 15.6,
+// 37 of 24^3 16.5 / 17.5, but of 20^3, whose cubes are half empty, 14.4 / 12.0.
+// In FP32 the one-step kernel is nowhere far ahead: 16^3 1.7 / 2.6, 62^3 3.0 /
+// 6.0; forty of 32^3 11.3 / 13.4, 120 35.5 / 33.0, 480 121 / 138; of 62^3
+// sixteen 38.1 / 35.1, 64 127 / 141; of 48^3 64 62.7 / 70.5; and a small member
+// beside large ones 32 and 192 61 / 58, 32 and 200 73 / 82, 24 and 400 474 / 671.
 // Wider stencils gain at most 1.2x (radius 2, 62^3) and lose up to 2x: not built.
 int block3d_depth(const Context *c)
 {
@@ -178,16 +184,20 @@ int block3d_depth(const Context *c)
         stencil_radius_of(c) != 1)
         return 0;
     bool small = false;
-    uint64_t cubes = 0;
+    uint64_t cubes = 0, sites = 0;
     for (const Member &m : c->members) {
         small = small || !march2_supported(c, m.N);
         const uint64_t t = (uint64_t)((m.N + kCubeOut - 1) / kCubeOut);
         cubes += t * t * t;
+        sites += (uint64_t)m.L;
     }
-    const uint64_t grid = kMaxGridItems / kCubeItems;
-    const uint64_t most = (c->prec == AXS_FP64) ? std::min<uint64_t>(4 * (uint64_t)c->num_cu, grid)
-                                                : grid;
-    return (small && cubes <= most) ? kCubeDepth : 0;
+    if (!small || cubes * kCubeItems > kMaxGridItems) return 0;
+    if (c->prec == AXS_FP64) {
+        const uint64_t cus = (uint64_t)(c->num_cu > 0 ? c->num_cu : 1);
+        const uint64_t rounds = (cubes + cus - 1) / cus;
+        if (rounds > 4 || 4.1 * (double)rounds > 6.0 + 22e-6 * (double)sites) return 0;
+    }
+    return kCubeDepth;
 }
 
 int prepare_block3d(Context *c)
