@@ -964,6 +964,25 @@ int axs_powerspec_all(axs_ctx *ctx, int binning, int nbins, double *ks, double *
     return run_powerspec_all(&ctx->impl, binning, nbins, ks, pk, count);
 }
 
+// a launch shape as axs_get_kernel_config reports it
+static axs_kernel_config shape_of(const Context *c, const Tune &t)
+{
+    axs_kernel_config k;
+    k.kernel = t.kernel;
+    k.rows = (t.depth >= 2 || c->p.stencil_setting > 0) ? t.rtb
+                                                         : ((c->prec == AXS_FP32) ? t.rj32 : t.rj64);
+    k.chunk = (c->prec == AXS_FP32) ? t.ci32 : t.ci64;
+    k.depth = t.depth;
+    k.flags = t.flags;
+    return k;
+}
+
+static bool same_shape(const axs_kernel_config &a, const axs_kernel_config &b)
+{
+    return a.kernel == b.kernel && a.rows == b.rows && a.chunk == b.chunk && a.depth == b.depth &&
+           a.flags == b.flags;
+}
+
 int axs_set_kernel_config(axs_ctx *ctx, const axs_kernel_config *cfg)
 {
     if (!ctx || !cfg) {
@@ -1028,18 +1047,24 @@ int axs_set_kernel_config(axs_ctx *ctx, const axs_kernel_config *cfg)
             set_error("chunk %d does not divide N=%d", cfg->chunk, m.N);
             return AXS_ERR_INVALID_ARG;
         }
-    c->tune.kernel = cfg->kernel;
+    Tune t = c->tune;
+    t.kernel = cfg->kernel;
     if (depth >= 2 || RAD > 1)
-        c->tune.rtb = cfg->rows;
+        t.rtb = cfg->rows;
     else if (c->prec == AXS_FP32)
-        c->tune.rj32 = cfg->rows ? cfg->rows : 8;
+        t.rj32 = cfg->rows ? cfg->rows : 8;
     else
-        c->tune.rj64 = cfg->rows ? cfg->rows : 4;
-    c->tune.ci32 = cfg->chunk;
-    c->tune.ci64 = cfg->chunk;
-    c->tune.depth = depth;
-    c->tune.flags = cfg->flags;
-    c->tune.configured = true;
+        t.rj64 = cfg->rows ? cfg->rows : 4;
+    t.ci32 = cfg->chunk;
+    t.ci64 = cfg->chunk;
+    t.depth = depth;
+    t.flags = cfg->flags;
+    t.configured = true;
+    // the shape the context reports, written back, leaves it as it is, and the
+    // shape it was created with brings its automatic choices back
+    const axs_kernel_config want = shape_of(c, t);
+    if (same_shape(want, shape_of(c, c->tune))) return AXS_OK;
+    c->tune = same_shape(want, shape_of(c, c->tune_default)) ? c->tune_default : t;
     return AXS_OK;
 }
 
@@ -1049,13 +1074,7 @@ int axs_get_kernel_config(const axs_ctx *ctx, axs_kernel_config *cfg)
         set_error("null argument");
         return AXS_ERR_INVALID_ARG;
     }
-    const Context *c = &ctx->impl;
-    cfg->kernel = c->tune.kernel;
-    cfg->rows = (c->tune.depth >= 2 || c->p.stencil_setting > 0) ? c->tune.rtb
-                                     : ((c->prec == AXS_FP32) ? c->tune.rj32 : c->tune.rj64);
-    cfg->chunk = (c->prec == AXS_FP32) ? c->tune.ci32 : c->tune.ci64;
-    cfg->depth = c->tune.depth;
-    cfg->flags = c->tune.flags;
+    *cfg = shape_of(&ctx->impl, ctx->impl.tune);
     return AXS_OK;
 }
 

@@ -287,7 +287,9 @@ typedef struct axs_kernel_config {
                      built, else with one-step launches; every split gives
                      the same bits.  Small 2D lattices and sides below 64
                      run up to six steps per pass on kernels of their own,
-                     with the same bits, until a configuration is set.      */
+                     with the same bits, until a configuration other than
+                     the one the context reports is set; setting the one it
+                     was created with brings them back.                     */
     int flags;    /* AXS_MARCH_* bits                                       */
 } axs_kernel_config;
 
