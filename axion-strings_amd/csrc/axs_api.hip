@@ -435,11 +435,12 @@ static int create_impl(const axs_params *p, int n_members, const int *Ns, axs_ct
         set_error("stream/event creation failed");
         return fail(AXS_ERR_HIP);
     }
-    if (hipHostMalloc(&c->mail, std::max<size_t>(4096, (size_t)n_members * 16),
-                      hipHostMallocDefault) != hipSuccess) {
+    const size_t mail_b = std::max<size_t>(4096, ((size_t)n_members * 16 + 255) & ~(size_t)255);
+    if (hipHostMalloc(&c->mail, mail_b + kListDirect, hipHostMallocDefault) != hipSuccess) {
         set_error("pinned result buffer failed");
         return fail(AXS_ERR_OUT_OF_MEMORY);
     }
+    c->mail_list = (int32_t *)((char *)c->mail + mail_b);
     c->members.resize(n_members);
     for (int r = 0; r < n_members; ++r) {
         Member &m = c->members[r];

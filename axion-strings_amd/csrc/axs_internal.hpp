@@ -116,6 +116,9 @@ struct Member {
 struct FftPlan;
 struct HostPool;
 
+// coordinate lists up to this size reach the host without a copy
+constexpr size_t kListDirect = (size_t)256 << 10;
+
 // one member of an ensemble as seen by the one-launch-per-step kernels
 struct BatchMember {
     int N, nTj, nTk, CI;     // 3D march tiling (2D: N only)
@@ -181,9 +184,11 @@ struct Context {
     // the compaction's counts survive its growth)
     void *listbuf = nullptr;
     size_t listbuf_bytes = 0;
-    // pinned host memory that kernels write small results to (counts, sums),
-    // 4 KiB or two counters per member: read after a stream synchronisation
+    // pinned host memory that kernels write small results to, read after a
+    // stream synchronisation: counts and sums (4 KiB, or two counters per
+    // member), then kListDirect bytes for a short coordinate list
     void *mail = nullptr;
+    int32_t *mail_list = nullptr;
     // pinned host staging
     void *pinned = nullptr;
     size_t pinned_bytes = 0;

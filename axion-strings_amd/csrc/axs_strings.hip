@@ -765,8 +765,6 @@ int run_axion(Context *c, Member &m, double *out)
     return copy_to_host(c, out, d, (size_t)L * sizeof(double));
 }
 
-constexpr size_t kListDirect = (size_t)256 << 10;
-
 int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *count,
                 int64_t *num_cores)
 {
@@ -836,11 +834,8 @@ int run_strings(Context *c, Member &m, int32_t *coords, int64_t cap, int64_t *co
     // directly, which saves a copy's launch and wait (256^2: 8 us)
     const size_t list_b = (size_t)total * c->nd * sizeof(int32_t) + 256;
     const bool direct = list_b <= kListDirect && num_cores == nullptr;
-    if (direct)
-        AXS_TRY(ensure_pinned(c, kListDirect));
-    else
-        AXS_TRY(ensure_device(c, &c->listbuf, &c->listbuf_bytes, list_b));
-    int32_t *dlist = (int32_t *)(direct ? c->pinned : c->listbuf);
+    if (!direct) AXS_TRY(ensure_device(c, &c->listbuf, &c->listbuf_bytes, list_b));
+    int32_t *dlist = direct ? c->mail_list : (int32_t *)c->listbuf;
 
     if (total > 0) {
         auto kw = (c->nd == 2) ? strings_write_kernel<2> : strings_write_kernel<3>;
