@@ -262,8 +262,9 @@ int ensure_scratch(Context *c, size_t bytes);
 int ensure_device(Context *c, void **buf, size_t *have, size_t bytes);
 int ensure_pinned(Context *c, size_t bytes);
 // Bulk transfers (axs_transfer.hip).  A segment is L sites of site_bytes each
-// at dev; fn converts sites [lo, lo + n) between their staged bytes and the
-// caller's arrays, on several host threads at once.  Synchronous on return.
+// (1, 8 or 16) at dev, on a 16-byte boundary; fn converts sites [lo, lo + n)
+// between their staged bytes and the caller's arrays, on several host threads
+// at once.  Synchronous on return.
 struct Segment {
     void *dev;
     size_t site_bytes, L;

@@ -8,9 +8,10 @@
 // chunks travel; to the device, the threads pack chunks ahead of the copies.
 // The pinned memory is the ring (24 MiB at most), whatever the lattice's
 // size, where a staging copy of a whole array per field took as long to pin
-// as to send.  128^3 FP64, six arrays of 16.8 MB: read-back 3.3-4.1 -> 2.3 ms,
-// upload 3.6 -> 2.5 ms (slots of 1 or 2 MiB, or eight threads: 2.7-3.3 ms);
-// 1000^2, two arrays: 0.90 -> 0.42 ms.
+// as to send.  In ms, a staging copy per array and the runtime's copies / now:
+// six arrays of 128^3 up 3.5 / 2.1, back 4.6-6.5 / 2.6; of 256^3 22 / 16 and 24 /
+// 18; two of 1000^2 back 1.9 / 0.7 (slots of 1 or 2 MiB, or eight threads: up to
+// 20% more; of 8 MiB 2-5% less, but more to pin on a first call).
 #include <string.h>
 
 #include <algorithm>
@@ -152,6 +153,40 @@ void parallel_for(Context *c, size_t n, void (*fn)(size_t, size_t, void *), void
 
 namespace {
 
+// One chunk between a slot and its device array, 16 bytes a work-item and
+// round; n16 of them, then the last bytes one by one.  64 groups keep the link
+// full (52 GB/s either way at 4 MiB, as 256 do).  A kernel rather than a copy
+// command: in many contexts the runtime's copies of a chunk cost 130 us each
+// beside their transfer once both directions have been used, whatever the
+// host's load (a list of 743 MB 44 ms, against 30 in 64 MiB chunks and 19 now;
+// six arrays of 128^3, upload / read-back: 5.5 / 5.5 ms, 2.1 / 2.6 now).  Small
+// transfers, a chunk at a time, keep the copy command: 10 to 20 us less.
+__global__ void __launch_bounds__(256)
+chunk_copy_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst, uint32_t n16,
+                  uint32_t tail)
+{
+    // one contiguous eighth per XCD (work-groups are dealt to the eight in
+    // turn): each translates the host pages of its own part only
+    const uint32_t part = (n16 + 7) / 8, x = blockIdx.x & 7u;
+    const uint32_t lo = x * part, hi = lo + part < n16 ? lo + part : n16;
+    const uint32_t step = (gridDim.x / 8) * 256u;
+    for (uint32_t i = lo + (blockIdx.x >> 3) * 256u + threadIdx.x; i < hi; i += step)
+        dst[i] = src[i];
+    if (blockIdx.x == 0 && threadIdx.x < tail)
+        ((unsigned char *)(dst + n16))[threadIdx.x] =
+            ((const unsigned char *)(src + n16))[threadIdx.x];
+}
+
+// both ends on 16-byte boundaries (whole arrays, slots, whole slots into them)
+hipError_t copy_chunk(Context *c, void *dst, const void *src, size_t bytes)
+{
+    const uint32_t n16 = (uint32_t)(bytes / 16);
+    const uint32_t groups = 8 * std::max(1u, std::min(8u, (n16 + 2047) / 2048));
+    hipLaunchKernelGGL(chunk_copy_kernel, dim3(groups), dim3(256), 0, c->stream,
+                       (const uint4 *)src, (uint4 *)dst, n16, (uint32_t)(bytes % 16));
+    return hipGetLastError();
+}
+
 constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr int kSlots = 6;
 constexpr int kSlices = 16;                // pieces of a chunk that threads take
@@ -250,16 +285,16 @@ int transfer(Context *c, const Segment *segs, int nsegs, bool to_host)
     w.ring = (char *)c->pinned;
     for (int h = 0; h < w.slots; ++h)
         if (!c->stage_ev[h])
-            AXS_HIP_TRY(hipEventCreateWithFlags(&c->stage_ev[h], hipEventDisableTiming));
+            AXS_HIP_TRY(hipEventCreateWithFlags(
+                &c->stage_ev[h], hipEventDisableTiming | hipEventReleaseToSystem));
     p->start(pipe_worker, &w);
 
     auto copy = [&](size_t q) -> hipError_t {
         const Chunk &k = w.chunks[q];
         char *dev = (char *)k.seg->dev + k.lo * k.seg->site_bytes;
         const size_t nb = k.n * k.seg->site_bytes;
-        hipError_t e = to_host
-                           ? hipMemcpyAsync(w.slot(q), dev, nb, hipMemcpyDeviceToHost, c->stream)
-                           : hipMemcpyAsync(dev, w.slot(q), nb, hipMemcpyHostToDevice, c->stream);
+        hipError_t e = to_host ? copy_chunk(c, w.slot(q), dev, nb)
+                               : copy_chunk(c, dev, w.slot(q), nb);
         if (e == hipSuccess) e = hipEventRecord(c->stage_ev[q % (size_t)w.slots], c->stream);
         return e;
     };
