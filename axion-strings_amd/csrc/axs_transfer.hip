@@ -17,7 +17,9 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <memory>
 #include <mutex>
+#include <optional>
 #include <thread>
 #include <vector>
 
@@ -96,16 +98,33 @@ void destroy_pool(Context *c)
     c->pool = nullptr;
 }
 
-// the context's threads; null where none could be started
-static HostPool *pool_of(Context *c)
-{
-    std::lock_guard<std::mutex> lk(c->pool_mu);
-    if (!c->pool) {
-        const unsigned hw = std::thread::hardware_concurrency();
-        c->pool = new (std::nothrow) HostPool(hw ? std::min(hw, 12u) : 4u);
+// Threads for one job: the context's, or, while they are at work for another
+// caller (a read-back beside axs_snapshot_end on another host thread), some of
+// its own for as long as it lasts.  p is null where none could be started.
+struct PoolLease {
+    HostPool *p = nullptr;
+    explicit PoolLease(Context *c)
+    {
+        const unsigned hw = std::thread::hardware_concurrency(), n = hw ? std::min(hw, 12u) : 4u;
+        {
+            std::lock_guard<std::mutex> lk(c->pool_mu);
+            if (!c->pool) c->pool = new (std::nothrow) HostPool(n);
+            p = c->pool;
+        }
+        if (p && !p->threads.empty()) {
+            job = std::unique_lock<std::mutex>(p->job_mu, std::try_to_lock);
+            if (!job.owns_lock()) {
+                own.reset(new (std::nothrow) HostPool(n));
+                p = own.get();
+            }
+        }
+        if (p && p->threads.empty()) p = nullptr;
     }
-    return (c->pool && !c->pool->threads.empty()) ? c->pool : nullptr;
-}
+
+private:
+    std::unique_lock<std::mutex> job;
+    std::unique_ptr<HostPool> own;
+};
 
 namespace {
 
@@ -134,10 +153,13 @@ void for_worker(void *p)
 
 void parallel_for(Context *c, size_t n, void (*fn)(size_t, size_t, void *), void *arg)
 {
-    HostPool *p = (n < kForAlone) ? nullptr : pool_of(c);
-    std::unique_lock<std::mutex> job;
-    if (p) job = std::unique_lock<std::mutex>(p->job_mu, std::try_to_lock);
-    if (!p || !job.owns_lock()) {          // small, or the threads are at work for another caller
+    if (n < kForAlone) {
+        fn(0, n, arg);
+        return;
+    }
+    PoolLease lease(c);
+    HostPool *p = lease.p;
+    if (!p) {
         fn(0, n, arg);
         return;
     }
@@ -260,10 +282,10 @@ int transfer(Context *c, const Segment *segs, int nsegs, bool to_host)
     }
     size_t bytes = 0;
     for (const Chunk &k : w.chunks) bytes += k.n * k.seg->site_bytes;
-    HostPool *p = (bytes < kPipeBytes) ? nullptr : pool_of(c);
-    std::unique_lock<std::mutex> job;
-    if (p) job = std::unique_lock<std::mutex>(p->job_mu, std::try_to_lock);
-    if (!p || !job.owns_lock()) {
+    std::optional<PoolLease> lease;
+    if (bytes >= kPipeBytes) lease.emplace(c);
+    HostPool *p = lease ? lease->p : nullptr;
+    if (!p) {
         // one slot, this thread alone
         AXS_TRY(ensure_pinned(c, w.slot_bytes));
         for (const Chunk &k : w.chunks) {

@@ -2,6 +2,8 @@
 work-item and the last bytes one by one: round trips whose last chunk holds
 one, a few or all but one of a slot's sites, and byte copies (coordinate
 lists, the axion field) of every remainder of 16."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -43,4 +45,29 @@ def test_byte_copies(N):
     n, c = lat.strings()
     assert n == n_ref
     np.testing.assert_array_equal(c, c_ref)
+    lat.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_read_backs_beside_a_snapshot(precision):
+    # axs_snapshot_end unpacks on another host thread while this one reads the
+    # state back: whichever comes second brings threads of its own
+    N = 128
+    rng = np.random.default_rng(5)
+    a = rng.standard_normal((6, N ** 3))
+    lat = axs.Lattice(3, N, precision=precision)
+    lat.set_state(*a, tau=1.0)
+    ref = lat.get_state()
+    for _ in range(4):
+        lat.snapshot_begin(fields=("phi1", "phi2", "phidot1", "phidot2", "ker1", "ker2"))
+        got = {}
+        t = threading.Thread(target=lambda: got.update(lat.snapshot_end()[0]))
+        t.start()
+        for _ in range(3):
+            g = lat.get_state()
+            for k in ref:
+                np.testing.assert_array_equal(g[k], ref[k], err_msg=k)
+        t.join()
+        for k in ref:
+            np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
     lat.close()
