@@ -794,6 +794,11 @@ fft_y_kernel(const double2 *__restrict__ ya, double2 *__restrict__ yb,
     }
 }
 
+// a wave's accumulator of a bin: a plain double (fft_bin_kernel) or a compensated
+// pair (any_bin_kernel)
+__device__ __forceinline__ void bin_add(double &a, double v) { a += v; }
+__device__ __forceinline__ void bin_add(KahanP &a, double v) { kaddp(a, v); }
+
 // C chunks of 64 frequencies fx = f0 + 64 c + lane of one transformed row, its
 // modes fx and -fx summed first (one |k|, one bin): C segmented scans side by side,
 // then the runs' sums into the wave's accumulators, chunk by chunk.  The scan's
@@ -801,11 +806,11 @@ fft_y_kernel(const double2 *__restrict__ ya, double2 *__restrict__ yb,
 // half the chunks and two chains at once took a linear-bin call from 12.7 to 11.5
 // ms at 1024^3, 1535 to 1431 us at 512^3, 1174 to 1085 at 400^3, 4191 to 3900 at
 // 640^3 and a batch of 32 x 64^3 from 253 to 235; four chains at once no further.
-template <int C>
+template <int C, class A>
 __device__ __forceinline__ void bin_chunks(const double2 *rb, int N, int half, int f0, int lane,
                                            uint64_t upto, uint32_t r2, uint32_t top, double w,
                                            int nbins, const uint16_t *shell, const uint32_t *hi2,
-                                           double *wacc)
+                                           A *wacc)
 {
     int b[C];
     uint32_t k2[C], hi[C];
@@ -876,14 +881,15 @@ __device__ __forceinline__ void bin_chunks(const double2 *rb, int N, int half, i
     }
 #pragma unroll
     for (int c = 0; c < C; ++c)
-        if (last[c] && b[c] >= 0 && b[c] < nbins) wacc[b[c]] += v[c];
+        if (last[c] && b[c] >= 0 && b[c] < nbins) bin_add(wacc[b[c]], v[c]);
 }
 
 // the modes of one transformed row, r2 = |k|^2 of its fixed components: two
 // chunks at a time while both hold a mode inside |k| < N/2
+template <class A>
 __device__ __forceinline__ void bin_row(const double2 *rb, int N, int half, int lane, uint64_t upto,
                                         uint32_t r2, uint32_t top, double w, int nbins,
-                                        const uint16_t *shell, const uint32_t *hi2, double *wacc)
+                                        const uint16_t *shell, const uint32_t *hi2, A *wacc)
 {
     int f0 = 0;
     for (; f0 + 64 < half && r2 + (uint32_t)((f0 + 64) * (f0 + 64)) < top; f0 += 128)
@@ -1328,12 +1334,13 @@ any_y_kernel(AnyGeom g, const double2 *__restrict__ ya, double2 *__restrict__ yb
     }
 }
 
-// last pass with the binning, as fft_bin_kernel
+// last pass with the binning, as fft_bin_kernel, but each wave's bin sums are
+// compensated pairs, as bin_scan_kernel's
 // (LDS: the group's rows, the twiddles, then the bins' sums and tables)
 static size_t any_bin_lds(int N, int R, int waves, int nbins, bool twl)
 {
     return ((size_t)R * any_ls(N) + (twl ? (size_t)N : 0)) * sizeof(double2) +
-           (size_t)waves * nbins * sizeof(double) + (size_t)nbins * 4 + (size_t)(N / 2) * 2;
+           (size_t)waves * nbins * sizeof(KahanP) + (size_t)nbins * 4 + (size_t)(N / 2) * 2;
 }
 
 template <int ND, int PTS, bool TWL>
@@ -1347,7 +1354,7 @@ any_bin_kernel(AnyGeom g, const double2 *__restrict__ y, const double2 *__restri
     const int N = g.N, half = N / 2, R = g.R, LS = any_ls(N);
     double2 *buf = reinterpret_cast<double2 *>(smem);
     double2 *twl = buf + R * LS;
-    double *acc = reinterpret_cast<double *>(twl + (TWL ? N : 0));     // [wave][bin]
+    KahanP *acc = reinterpret_cast<KahanP *>(twl + (TWL ? N : 0));     // [wave][bin]
     uint32_t *hi2 = reinterpret_cast<uint32_t *>(acc + W * nbins);
     uint16_t *shell = reinterpret_cast<uint16_t *>(hi2 + nbins);
     if (TWL) any_tw<THR>(twl, tw, N, 1);
@@ -1355,11 +1362,11 @@ any_bin_kernel(AnyGeom g, const double2 *__restrict__ y, const double2 *__restri
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int i = threadIdx.x; i < nbins; i += THR) {
         hi2[i] = hi2g[i];
-        for (int w = 0; w < W; ++w) acc[w * nbins + i] = 0.0;
+        for (int w = 0; w < W; ++w) acc[w * nbins + i] = KahanP{0.0, 0.0};
     }
     for (int i = threadIdx.x; i < half; i += THR) shell[i] = shellg[i];
     __syncthreads();
-    double *wacc = acc + wave * nbins;
+    KahanP *wacc = acc + wave * nbins;
     const double2 *yl = y + (size_t)blockIdx.y * g.nrows * N;
     const uint32_t top = (uint32_t)half * (uint32_t)half;
     const uint64_t upto = (2ull << lane) - 1;
@@ -1403,8 +1410,8 @@ any_bin_kernel(AnyGeom g, const double2 *__restrict__ y, const double2 *__restri
         __syncthreads();                             // before the next group's loads
     }
     for (int i = threadIdx.x; i < nbins; i += THR) {
-        KahanP a{acc[i], 0.0};
-        for (int w = 1; w < W; ++w) a = kmergep(a, KahanP{acc[w * nbins + i], 0.0});
+        KahanP a = acc[i];
+        for (int w = 1; w < W; ++w) a = kmergep(a, acc[w * nbins + i]);
         part[((size_t)blockIdx.y * nbins + i) * gridDim.x + blockIdx.x] = a;
     }
 }
@@ -1759,26 +1766,42 @@ static int any_group(const Context *c, int most, int nrows, int n)
     return (int)std::min<int64_t>(std::min(most, kAnyRows), std::min<int64_t>(spread, nrows));
 }
 
-// points and rows of the last pass's groups for rows of N points (the order of the
-// bins' sums, so the same for one spectrum and a batch), and the LDS it may take; the twiddles go to LDS where a group's rows leave room
+// The last pass's groups for rows of N points (their order is the order of the
+// bins' sums, so the same for one spectrum and a batch) and the LDS they may
+// take: two a CU at least, the twiddles in it where that leaves room
 static int any_bin_pts(int N) { return N > 2048 ? 4096 : 2048; }
-static int any_bin_rows(const Context *c, int N)
+constexpr size_t kAnyBinLds = 80 * 1024, kCuLds = 160 * 1024;
+
+// rows of a group: as many as its points hold, or fewer where more groups then
+// fit a CU and more rows are in flight (with the bins' pairs in the LDS a linear
+// call at 200^3 209 -> 203 us, 250^3 382 -> 374, 300^3 604 -> 587, 640^3 4.24 -> 4.01 ms)
+static int any_bin_rows(const Context *c, int N, int nbins)
 {
-    const int nrows = (c->nd == 3) ? N / 2 * N : N / 2;
-    return std::min(nrows, std::max(any_group(c, any_bin_pts(N) / N, nrows, 1),
-                                    std::min(512 / N, kAnyRows)));
+    const int nrows = (c->nd == 3) ? N / 2 * N : N / 2, waves = any_bin_pts(N) / 16 / 64;
+    const int most = std::min(nrows, std::max(any_group(c, any_bin_pts(N) / N, nrows, 1),
+                                              std::min(512 / N, kAnyRows)));
+    int best = most;
+    size_t flight = 0;
+    for (int R = most; R >= std::max(1, most / 2); --R) {
+        const size_t groups = kCuLds / any_bin_lds(N, R, waves, nbins, true);
+        const size_t n = std::min<size_t>(groups, 4) * (size_t)R;
+        if (n >= flight) {
+            flight = n;
+            best = R;
+        }
+    }
+    return best;
 }
-constexpr size_t kAnyBinLds = 64 * 1024;
 
 // Sides the run-time transform takes: those whose rows, their bins' sums and
-// tables fit the last pass's LDS (2D linear bins to N of about 2000)
+// tables fit the LDS (2D linear bins to N of 1285, where B.scan ends)
 static bool any_fft_ok(const Context *c, int N, const BinLayout &B)
 {
     if (c->pk_rocfft || N < 16 || N > (c->nd == 3 ? 1024 : 4096) || !B.scan) return false;
     AnyPlan p;
     if (!any_plan(N, p) || !any_plan(N / 2, p)) return false;
-    const int pts = any_bin_pts(N);
-    return any_bin_lds(N, any_bin_rows(c, N), pts / 16 / 64, B.nbins, false) <= kAnyBinLds;
+    const int waves = any_bin_pts(N) / 16 / 64;
+    return any_bin_lds(N, any_bin_rows(c, N, B.nbins), waves, B.nbins, false) <= kAnyBinLds;
 }
 
 // The n spectra of side N by the run-time transform (any_fft_ok).
@@ -1801,7 +1824,7 @@ static int pk_raw_any(Context *c, const PkSrc *srcs, int n, int N, const BinLayo
     y.GI = (N + y.R - 1) / y.R;
     y.R = (N + y.GI - 1) / y.GI;                    // groups of equal size
     x.nrows = (c->nd == 3) ? M * N : M;
-    x.R = any_bin_rows(c, N);
+    x.R = any_bin_rows(c, N, B.nbins);
     z.mR = magic_of((uint32_t)z.R);
     y.mR = magic_of((uint32_t)y.R);
     const uint32_t groups = ((uint32_t)x.nrows + x.R - 1) / (uint32_t)x.R;

@@ -209,7 +209,9 @@ int axs_member_energy_noalloc(axs_ctx *ctx, int member, double out[3]);
  * member `member`: AXS_BIN_LINEAR gives the reference's N/2 unit-width bins
  * (nbins ignored; arrays need N/2 entries); AXS_BIN_LOG gives nbins log bins
  * with pk the mean |F|^2 per mode.  ks, pk, count: one entry per bin.  Empty
- * bins have count 0.  FP64 transform, bins in compensated FP64.            */
+ * bins have count 0.  FP64 transform; bin sums in FP64, compensated (power-
+ * of-two sides from 128 on: each wave's own sums plain, their merge
+ * compensated).                                                            */
 int axs_member_powerspec(axs_ctx *ctx, int member, int binning, int nbins,
                          double *ks, double *pk, int32_t *count);
 int axs_powerspec(axs_ctx *ctx, int binning, int nbins,
