@@ -1011,13 +1011,14 @@ fft_bin_kernel(const double2 *__restrict__ y, const double2 *__restrict__ tw, in
 // sides, gained 7 to 14 % at 300^3, 500^3 and
 // 900^3, nothing at 200^3, 320^3 and 400^3, and lost 3 % at 640^3: not taken.
 // Against rocFFT, packing and bin_scan_kernel, a linear-bin call of the FP32
-// form, the same state (us): 2D 100 54 / 96, 250 57 / 102, 600 68 / 141, 1000
-// 85 / 186; 3D 48 81 / 95, 100 106 / 117, 200 205 / 209, 300 597 / 749, 400
-// 1083 / 1572, 500 2262 / 3093, 640 3850 / 6273, 768 7295 / 10354, 900 15097 /
-// 17206; batches 3D 64 x 48 252 / 291, 32 x 64 231 / 233, 16 x 96 327 / 323, but
-// 256 x 16 239 / 213; and a context's first call of a side 0.2 to 17 ms against 16
-// to 300 ms, most of it rocFFT's plan.  A bin's error against extended precision:
-// 2.7e-15 rms at 400^3 (rocFFT 3.2e-15), 1.1e-14 at 48^3 (3.0e-14).
+// form, the same state (us): 2D 48 55 / 94, 250 59 / 102, 600 69 / 142, 1000 85 /
+// 184; 3D 48 82 / 95, 100 104 / 112, 200 201 / 210, 300 590 / 730, 400 1068 /
+// 1560, 500 2210 / 3090, 640 4000 / 6270, 768 7050 / 10600, 900 14640 / 17150;
+// batches 3D 256 x 16 218 / 211, 64 x 32 132 / 137, 128 x 32 187 / 198, 64 x 48
+// 237 / 259, 32 x 64 233 / 231, but 32 x 72 303 / 280, 16 x 96 320 / 313, 16 x 100
+// 362 / 338; and a context's first call of a side 0.3 to 17 ms against 16 to 300 ms,
+// most of it rocFFT's plan.  A bin's error against extended precision, rms: 2.7e-15
+// at 400^3 (rocFFT 3.2e-15), 1.1e-14 at 48^3 (3.0e-14).
 struct AnyPlan {
     int L = 0, stages = 0;
     int rad[12], ns[12];               // radix, product of the earlier radices
@@ -1182,6 +1183,7 @@ __device__ __forceinline__ void any_rows(double2 *buf, const double2 *__restrict
 // points of a group's rows in LDS, with the rows' padding: R rows of L points,
 // R L <= PTS and R <= kAnyRows, take R (L + L/16 + 1)
 constexpr int kAnyRows = 128;
+constexpr int kAnySmall = 32;          // sides whose Y pass runs in groups of kAnySmall^2
 template <int PTS>
 constexpr int any_lds() { return PTS + PTS / 16 + kAnyRows; }
 
@@ -1306,26 +1308,31 @@ __device__ __forceinline__ void any_load(double2 *buf, const double2 *__restrict
     }
 }
 
-// Y pass (3D): rows Y[b][i][k_z][*] of R consecutive i; Y'[b][k_z][k_j][i]
-__global__ void __launch_bounds__(kFftPtsY / 16)
+// Y pass (3D): rows Y[b][i][k_z][*] of R consecutive i; Y'[b][k_z][k_j][i].
+// Groups of PTS points: a side up to 32 has at most 1024 to one (b, k_z), and
+// fills an eighth of the large groups' LDS, one of which a CU takes; in groups of
+// its own size a batch of 256 x 16^3 spectra falls from 247 to 218 us, 64 x 32^3 159
+// to 132, 128 x 32^3 241 to 187.
+template <int PTS>
+__global__ void __launch_bounds__(PTS / 16)
 any_y_kernel(AnyGeom g, const double2 *__restrict__ ya, double2 *__restrict__ yb,
              const double2 *__restrict__ tw)
 {
-    constexpr int THR = kFftPtsY / 16;
-    __shared__ double2 buf[any_lds<kFftPtsY>()];
-    __shared__ double2 twl[1024];
+    constexpr int THR = PTS / 16;
+    __shared__ double2 buf[any_lds<PTS>()];
+    __shared__ double2 twl[PTS < kFftPtsY ? kAnySmall : 1024];
     any_tw<THR>(twl, tw, g.N, 1);
     const int N = g.N, M = N / 2, R = g.R, LS = any_ls(N);
     const uint32_t ig = blockIdx.x % (uint32_t)g.GI, t = blockIdx.x / (uint32_t)g.GI;
     const uint32_t kz = t % (uint32_t)M, b = t / (uint32_t)M;
     const int i0 = (int)ig * R, rows = (N - i0 < R) ? N - i0 : R;
     const double2 *src = ya + (((size_t)b * N + i0) * M + kz) * N;
-    any_load<kFftPtsY / THR, THR>(buf, src, rows * N, (size_t)M * N, g, LS);
+    any_load<16, THR>(buf, src, rows * N, (size_t)M * N, g, LS);
     __syncthreads();
     any_rows<THR>(buf, twl, 1, g.p, LS, rows);
     double2 *dst = yb + ((size_t)b * M + kz) * N * N + i0;
 #pragma unroll 4
-    for (int q = 0; q < kFftPtsY / THR; ++q) {
+    for (int q = 0; q < 16; ++q) {
         const int e = threadIdx.x + q * THR;
         if (e < R * N) {
             const int kj = fast_div(e, g.mR), r = e - kj * R;
@@ -1820,7 +1827,8 @@ static int pk_raw_any(Context *c, const PkSrc *srcs, int n, int N, const BinLayo
     any_plan(N, x.p);
     z.nrows = (c->nd == 3) ? N * N : N;
     z.R = any_group(c, kFftPts / M, z.nrows, n);
-    y.R = any_group(c, kFftPtsY / N, N, n * M);
+    const bool small = N <= kAnySmall;
+    y.R = any_group(c, (small ? kAnySmall * kAnySmall : kFftPtsY) / N, N, n * M);
     y.GI = (N + y.R - 1) / y.R;
     y.R = (N + y.GI - 1) / y.GI;                    // groups of equal size
     x.nrows = (c->nd == 3) ? M * N : M;
@@ -1840,8 +1848,14 @@ static int pk_raw_any(Context *c, const PkSrc *srcs, int n, int N, const BinLayo
     if (c->nd == 3) {
         hipLaunchKernelGGL((any_z_kernel<3, true>), dim3(gz, (unsigned)n), dim3(kFftThr), 0,
                            c->stream, z, t.src, p->ya, p->tw);
-        hipLaunchKernelGGL(any_y_kernel, dim3((unsigned)n * M * y.GI), dim3(kFftPtsY / 16), 0,
-                           c->stream, y, p->ya, p->yb, p->tw);
+        const unsigned gy = (unsigned)n * M * y.GI;
+        if (small)
+            hipLaunchKernelGGL(any_y_kernel<kAnySmall * kAnySmall>, dim3(gy),
+                               dim3(kAnySmall * kAnySmall / 16), 0, c->stream, y, p->ya, p->yb,
+                               p->tw);
+        else
+            hipLaunchKernelGGL(any_y_kernel<kFftPtsY>, dim3(gy), dim3(kFftPtsY / 16), 0,
+                               c->stream, y, p->ya, p->yb, p->tw);
         last = p->yb;
     } else {
         auto kz = (M <= 512) ? any_z_kernel<2, true> : any_z_kernel<2, false>;
