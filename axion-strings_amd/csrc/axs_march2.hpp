@@ -120,21 +120,20 @@ __device__ __forceinline__ void tile_of(uint32_t t, const TBGeom &g, int &tj, in
 
 // LDS sets of the levels' planes.  Two, where they fit: the next plane goes to
 // the other set, and one barrier a plane orders both.  One: a barrier before the
-// writes and one after.  Two are faster on every lattice tried (us a step: FP32
-// 512^3 260 -> 245, 640^3 460 -> 441, 896^3 1187 -> 1148, the 48-lattice ensemble
-// 720 -> 712; FP64 128^3 22.1 -> 21.1, 256^3 147 -> 143, 640^3 1.82 -> 1.74 ms,
-// 1024^3 7.17 -> 7.05 ms) but one: FP32 rows of a whole number of 16 KiB
-// (1024^3), whose lines of one column fall on the same memory channels; there
-// the freer waves spread the work-groups' planes apart, 1.77 -> 1.86 ms.
+// writes and one after.  Two are faster on the lattices tried (us a step: FP32
+// 512^3 260 -> 245, 704^3 607 -> 587, 768^3 742 -> 717, 896^3 1201 -> 1177, 1000^3
+// 1626 -> 1552, 1040^3 1854 -> 1774, 1152^3 2517 -> 2431, 1280^3 3603 -> 3562, the
+// 48-lattice ensemble 720 -> 712; FP64 128^3 22.1 -> 21.1, 256^3 147 -> 143, 640^3
+// 1.82 -> 1.74 ms, 1024^3 7.17 -> 7.05 ms) but for 7-point FP32 passes over one
+// lattice whose rows are a whole number of 16 KiB (16 N bytes): there the lines
+// of a column repeat on the same memory channels, and how the work-groups' waves
+// are spread decides.  24 lattices of 1024^3 each, ms a step: one set 1.69-1.98,
+// median 1.77; two 1.64-2.01, median 1.91, at the same bytes fetched and the same
+// L2 misses.  Sixth order (5.08 -> 4.95) and ensembles (two of 1024^3 4.08 / 4.05,
+// work-groups in another order) take two there too.
 template <class T, int D, int W, int R, int RAD>
 constexpr bool kTwoSets = 2 * D * 2 * (W * R + 2 * RAD) * kTBW * (int)sizeof(T) <= 160 * 1024;
-template <class Tr, int D, int W, int R, int RAD>
-inline bool two_sets(int N)
-{
-    using T = typename Tr::T;
-    if (!kTwoSets<T, D, W, R, RAD>) return false;
-    return !std::is_same<T, float>::value || (size_t)N * 16 % 16384 != 0;
-}
+inline bool aliased_rows(int N) { return (size_t)N * 16 % 16384 == 0; }
 
 // x_l of the plane level l works on: the ER loaded rows plus RAD padding
 // rows above and below, so that the neighbour reads of the rim rows and
@@ -491,14 +490,15 @@ struct SingleLaunch {
         g.CI = multi_chunk(c, N, TJ, TK, D * RAD);
         const uint32_t nb = (uint32_t)g.nTj * (uint32_t)g.nTk * (uint32_t)((N + g.CI - 1) / g.CI);
         tile_order<Tr>(g);
-        if constexpr (kTwoSets<typename Tr::T, D, W, R, RAD>) {
-            if (two_sets<Tr, D, W, R, RAD>(N)) {
+        constexpr bool fit = kTwoSets<typename Tr::T, D, W, R, RAD>;
+        if constexpr (fit && std::is_same<Tr, F32Form>::value && RAD == 1) {
+            if (aliased_rows(N))
+                launch<W, R, 1>(nb, g);
+            else
                 launch<W, R, 2>(nb, g);
-                return AXS_OK;
-            }
+        } else {
+            launch<W, R, fit ? 2 : 1>(nb, g);
         }
-        if constexpr (std::is_same<Tr, F32Form>::value || !kTwoSets<typename Tr::T, D, W, R, RAD>)
-            launch<W, R, 1>(nb, g);
         return AXS_OK;
     }
     template <int W, int R, int SETS>
@@ -522,14 +522,7 @@ struct BatchLaunch {
     template <int W, int R>
     int run()
     {
-        if constexpr (kTwoSets<typename Tr::T, D, W, R, RAD>) {
-            bool two = true;
-            for (const Member &m : c->members) two = two && two_sets<Tr, D, W, R, RAD>(m.N);
-            if (two) return launch<W, R, 2>();
-        }
-        if constexpr (std::is_same<Tr, F32Form>::value || !kTwoSets<typename Tr::T, D, W, R, RAD>)
-            return launch<W, R, 1>();
-        return AXS_OK;
+        return launch<W, R, kTwoSets<typename Tr::T, D, W, R, RAD> ? 2 : 1>();
     }
     template <int W, int R, int SETS>
     int launch()
