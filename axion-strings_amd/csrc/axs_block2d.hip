@@ -33,23 +33,6 @@ constexpr int blk_depth(int RAD) { return RAD == 1 ? 6 : 8 / RAD; }
 constexpr int blk_cols(int RAD) { return kBlkSide - 2 * blk_depth(RAD) * RAD; }
 constexpr int blk_rows(int RAD, int R) { return kBlkSide * R - 2 * blk_depth(RAD) * RAD; }
 
-template <class Tr>
-__device__ __forceinline__ typename Tr::In blk_in(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(const fvec4 *)p[PHI]};
-    else
-        return {(const dvec2 *)p[PHI], (const dvec2 *)p[VEL], (const dvec2 *)p[KER]};
-}
-template <class Tr>
-__device__ __forceinline__ typename Tr::Out blk_out_arrays(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(fvec4 *)p[PHI]};
-    else
-        return {(dvec2 *)p[PHI], (dvec2 *)p[VEL], (dvec2 *)p[KER]};
-}
-
 // d <= blk_depth(RAD) steps of block `t` of lattice m; R consecutive rows per
 // work-item, a region of 32 columns and 32 R rows
 template <class Tr, int RAD, int R>
@@ -79,7 +62,7 @@ __device__ __forceinline__ void block2d_tile(const BatchMember &m, const uint32_
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         q[r] = (uint32_t)wrap(j0 - H + cj + r) * (uint32_t)N + qi;
-        Tr::fetch(blk_in<Tr>(m.in), q[r], raw[r]);
+        Tr::fetch(form_in<Tr>(m.in), q[r], raw[r]);
     }
     const typename Tr::Vc vc = Tr::vconst(sc.s[0]);
     T x[R], y[R];
@@ -145,7 +128,7 @@ __device__ __forceinline__ void block2d_tile(const BatchMember &m, const uint32_
     for (int r = 0; r < R; ++r) {
         const int e = cj + r;
         if (icol && e >= H && e < H + TJ && j0 + e - H < N)
-            Tr::store(blk_out_arrays<Tr>(m.out), q[r], x[r], y[r], own[r]);
+            Tr::store(form_out<Tr>(m.out), q[r], x[r], y[r], own[r]);
     }
 }
 
@@ -190,9 +173,10 @@ static uint64_t block2d_tiles(const Context *c, int R)
 // height overhead: FP64 1000^2 6.8 -> 5.9 us a step, fourth order 13.6 -> 10.1;
 // FP32 3.7 -> 2.7.  FP64 radius 3 and 4 keep one (two rows of their sums leave
 // one group per CU: 17.3 against 19.1 us at 1000^2, radius 3).
+constexpr bool two_rows_built(bool f64, int RAD) { return !f64 || RAD <= 2; }
 static int block2d_rows(const Context *c)
 {
-    if (c->prec == AXS_FP64 && stencil_radius_of(c) > 2) return 1;
+    if (!two_rows_built(c->prec == AXS_FP64, stencil_radius_of(c))) return 1;
     return block2d_tiles(c, 1) <= 2 * (uint64_t)c->num_cu ? 1 : 2;
 }
 
@@ -311,10 +295,9 @@ static void launch_rad(Context *c, int src, const StepScalars *s, int d)
         else
             sc.s[l] = s[l];
     }
-    if (c->blk.key == 2)
-        launch_rows<Tr, RAD, 2>(c, src, sc, d);
-    else
-        launch_rows<Tr, RAD, 1>(c, src, sc, d);
+    if constexpr (two_rows_built(!std::is_same<Tr, F32Form>::value, RAD))
+        if (c->blk.key == 2) return launch_rows<Tr, RAD, 2>(c, src, sc, d);
+    launch_rows<Tr, RAD, 1>(c, src, sc, d);
 }
 
 template <class Tr>

@@ -30,23 +30,6 @@ constexpr int kCubeItems = kCubeSide * kCubeSide * kCubeSide / kCubeRows;
 constexpr int kCubeDepth = 4;                       // most steps of a pass
 constexpr int kCubeOut = kCubeSide - 2 * kCubeDepth;
 
-template <class Tr>
-__device__ __forceinline__ typename Tr::In cube_in(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(const fvec4 *)p[PHI]};
-    else
-        return {(const dvec2 *)p[PHI], (const dvec2 *)p[VEL], (const dvec2 *)p[KER]};
-}
-template <class Tr>
-__device__ __forceinline__ typename Tr::Out cube_arrays(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(fvec4 *)p[PHI]};
-    else
-        return {(dvec2 *)p[PHI], (dvec2 *)p[VEL], (dvec2 *)p[KER]};
-}
-
 // d <= kCubeDepth steps of cube `t` of lattice m
 template <class Tr>
 __device__ __forceinline__ void block3d_tile(const BatchMember &m, const uint32_t t, const int d,
@@ -80,7 +63,7 @@ __device__ __forceinline__ void block3d_tile(const BatchMember &m, const uint32_
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         q[r] = (uint32_t)wrap(i0 - H + ci + r) * un * un + col;
-        Tr::fetch(cube_in<Tr>(m.in), q[r], raw[r]);
+        Tr::fetch(form_in<Tr>(m.in), q[r], raw[r]);
     }
     const typename Tr::Vc vc = Tr::vconst(sc.s[0]);
     T x[R], y[R];
@@ -136,7 +119,7 @@ __device__ __forceinline__ void block3d_tile(const BatchMember &m, const uint32_
     for (int r = 0; r < R; ++r) {
         const int e = ci + r;
         if (inner && e >= H && e < H + TS && i0 + e - H < N)
-            Tr::store(cube_arrays<Tr>(m.out), q[r], x[r], y[r], own[r]);
+            Tr::store(form_out<Tr>(m.out), q[r], x[r], y[r], own[r]);
     }
 }
 

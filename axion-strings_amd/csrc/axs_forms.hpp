@@ -18,6 +18,8 @@
 // so a pass of D levels gives the bits of D one-step launches.
 #pragma once
 
+#include <type_traits>
+
 #include "axs_internal.hpp"
 #include "axs_lattice.hpp"
 
@@ -169,5 +171,23 @@ struct F64FormT {
         store_nt(o.ker + q, w.k);
     }
 };
+
+// the form's array views from a member-table entry (device) or a member (host)
+template <class Tr>
+__host__ __device__ __forceinline__ typename Tr::In form_in(void *const *p)
+{
+    if constexpr (std::is_same<Tr, F32Form>::value)
+        return {(const fvec4 *)p[PHI]};
+    else
+        return {(const dvec2 *)p[PHI], (const dvec2 *)p[VEL], (const dvec2 *)p[KER]};
+}
+template <class Tr>
+__host__ __device__ __forceinline__ typename Tr::Out form_out(void *const *p)
+{
+    if constexpr (std::is_same<Tr, F32Form>::value)
+        return {(fvec4 *)p[PHI]};
+    else
+        return {(dvec2 *)p[PHI], (dvec2 *)p[VEL], (dvec2 *)p[KER]};
+}
 
 }  // namespace axs

@@ -402,24 +402,6 @@ marchd_kernel(TBGeom g, typename Tr::In in, typename Tr::Out out,
     marchd_tile<Tr, D, W, R, RAD, PF, SETS>(g.N, g.CI, tj, tk, ch, in, out, sc, X);
 }
 
-// the form's array views from a member-table entry (device) or a member (host)
-template <class Tr>
-__host__ __device__ __forceinline__ typename Tr::In form_in(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(const fvec4 *)p[PHI]};
-    else
-        return {(const dvec2 *)p[PHI], (const dvec2 *)p[VEL], (const dvec2 *)p[KER]};
-}
-template <class Tr>
-__host__ __device__ __forceinline__ typename Tr::Out form_out(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(fvec4 *)p[PHI]};
-    else
-        return {(dvec2 *)p[PHI], (dvec2 *)p[VEL], (dvec2 *)p[KER]};
-}
-
 // Ensemble form: one persistent launch for every member.  Work items are
 // the (member, tile, chunk) triples, members in order, tiles k fastest;
 // work-group b takes items b, b + gridDim.x, ...  The barrier that ends a

@@ -197,23 +197,6 @@ __device__ __forceinline__ void march2d_strip(const int N, const int chunk, cons
     for (; it < CJ; ++it) row_step(it);
 }
 
-template <class Tr>
-__device__ __forceinline__ typename Tr::In strip_in(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(const fvec4 *)p[PHI]};
-    else
-        return {(const dvec2 *)p[PHI], (const dvec2 *)p[VEL], (const dvec2 *)p[KER]};
-}
-template <class Tr>
-__device__ __forceinline__ typename Tr::Out strip_out(void *const *p)
-{
-    if constexpr (std::is_same<Tr, F32Form>::value)
-        return {(fvec4 *)p[PHI]};
-    else
-        return {(dvec2 *)p[PHI], (dvec2 *)p[VEL], (dvec2 *)p[KER]};
-}
-
 // one work item per wave: (member, strip, chunk) from the member table
 template <class Tr, int D, int RAD, bool PF>
 __global__ void __launch_bounds__(64 * kWaves2D)
@@ -237,8 +220,8 @@ march2d_kernel(const BatchMember *__restrict__ mem, int n_members, uint32_t n_it
         const uint32_t t = item - m.item_begin;
         const int ti = (int)(t % (uint32_t)m.nTj);
         const int ch = (int)(t / (uint32_t)m.nTj);
-        march2d_strip<Tr, D, RAD, PF>(m.N, m.CI, ti, ch, strip_in<Tr>(m.in),
-                                      strip_out<Tr>(m.out), sc);
+        march2d_strip<Tr, D, RAD, PF>(m.N, m.CI, ti, ch, form_in<Tr>(m.in),
+                                      form_out<Tr>(m.out), sc);
     }
 }
 
