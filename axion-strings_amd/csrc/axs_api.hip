@@ -235,7 +235,7 @@ Context::~Context()
 {
     if (stream) (void)hipStreamSynchronize(stream);
     destroy_snapshot(this);
-    destroy_pool(this);
+    release_pool(this);
     destroy_plans(this);
     destroy_inverse_plans(this);
     destroy_spec_plans(this);

@@ -114,7 +114,6 @@ struct Member {
 };
 
 struct FftPlan;
-struct HostPool;
 
 // coordinate lists up to this size reach the host without a copy
 constexpr size_t kListDirect = (size_t)256 << 10;
@@ -193,10 +192,7 @@ struct Context {
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
 
-    // host threads of the bulk transfers (axs_transfer.hip), started on first
-    // use (snapshot_end may be the first, from another host thread)
-    HostPool *pool = nullptr;
-    std::mutex pool_mu;
+    bool pool_user = false;       // holds the shared host threads (axs_transfer.hip)
 
     // asynchronous snapshot (axs_snapshot.hip): device staging copy made on
     // `stream`, device-to-host copy on `copy_stream`
@@ -274,11 +270,11 @@ struct Segment {
 int transfer(Context *c, const Segment *segs, int nsegs, bool to_host);
 // device-to-host copy of `bytes` into a caller's (pageable) buffer
 int copy_to_host(Context *c, void *dst, const void *src, size_t bytes);
-// host-side parallel loop over [0, n) in contiguous pieces on the context's
+// host-side parallel loop over [0, n) in contiguous pieces on the shared
 // threads (small n: on the calling thread)
 void parallel_for(Context *c, size_t n, void (*fn)(size_t begin, size_t end, void *arg),
                   void *arg);
-void destroy_pool(Context *c);
+void release_pool(Context *c);
 
 // ---------------------------------------------------------------------------
 // launchers (return AXS_OK or an error code)

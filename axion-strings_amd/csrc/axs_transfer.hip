@@ -27,8 +27,8 @@
 
 namespace axs {
 
-// host threads of one context, started by its first large transfer and ended
-// with the context
+// host threads for the bulk work of all contexts, started by the first large
+// transfer and ended with the last context that used them
 struct HostPool {
     std::mutex job_mu;                     // one job at a time
     std::mutex mu;
@@ -92,24 +92,40 @@ struct HostPool {
     }
 };
 
-void destroy_pool(Context *c)
+static std::mutex g_pool_mu;
+static HostPool *g_pool = nullptr;
+static int g_pool_users = 0;               // contexts with pool_user set
+
+void release_pool(Context *c)
 {
-    delete c->pool;
-    c->pool = nullptr;
+    HostPool *last = nullptr;
+    {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        if (c->pool_user && --g_pool_users == 0) {
+            last = g_pool;
+            g_pool = nullptr;
+        }
+        c->pool_user = false;
+    }
+    delete last;
 }
 
-// Threads for one job: the context's, or, while they are at work for another
-// caller (a read-back beside axs_snapshot_end on another host thread), some of
-// its own for as long as it lasts.  p is null where none could be started.
+// Threads for one job: the shared ones, or, while they are at work for another
+// caller (a read-back beside axs_snapshot_end, another context), some of its own
+// for as long as it lasts.  p is null where none could be started.
 struct PoolLease {
     HostPool *p = nullptr;
     explicit PoolLease(Context *c)
     {
         const unsigned hw = std::thread::hardware_concurrency(), n = hw ? std::min(hw, 12u) : 4u;
         {
-            std::lock_guard<std::mutex> lk(c->pool_mu);
-            if (!c->pool) c->pool = new (std::nothrow) HostPool(n);
-            p = c->pool;
+            std::lock_guard<std::mutex> lk(g_pool_mu);
+            if (!g_pool) g_pool = new (std::nothrow) HostPool(n);
+            if (g_pool && !c->pool_user) {
+                c->pool_user = true;
+                ++g_pool_users;
+            }
+            p = g_pool;
         }
         if (p && !p->threads.empty()) {
             job = std::unique_lock<std::mutex>(p->job_mu, std::try_to_lock);

@@ -2,6 +2,7 @@
 work-item and the last bytes one by one: round trips whose last chunk holds
 one, a few or all but one of a slot's sites, and byte copies (coordinate
 lists, the axion field) of every remainder of 16."""
+import os
 import threading
 
 import numpy as np
@@ -71,3 +72,25 @@ def test_read_backs_beside_a_snapshot(precision):
         for k in ref:
             np.testing.assert_array_equal(got[k], ref[k], err_msg=k)
     lat.close()
+
+
+def test_contexts_share_their_threads():
+    # each context's transfers are large enough to be shared among threads
+    N = 700
+    a = np.random.default_rng(6).standard_normal((4, N * N))
+    lats = []
+    for k in range(6):
+        lat = axs.Lattice(2, N)
+        lat.set_state(*a, tau=1.0)
+        g = lat.get_state()
+        np.testing.assert_array_equal(g["phi2"], a[1])
+        lats.append(lat)
+        if k == 0:
+            first = len(os.listdir("/proc/self/task"))
+    assert len(os.listdir("/proc/self/task")) < first + 4
+    lats[0].close()                     # the others go on with the same threads
+    lats[1].set_state(*-a, tau=1.0)
+    np.testing.assert_array_equal(lats[1].get_state()["phi1"], -a[0])
+    for lat in lats[1:]:
+        lat.close()
+    assert len(os.listdir("/proc/self/task")) < first
