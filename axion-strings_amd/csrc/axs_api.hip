@@ -495,8 +495,8 @@ static int create_impl(const axs_params *p, int n_members, const int *Ns, axs_ct
     }
     // several steps per pass unless configured otherwise (the fastest
     // shapes measured).  Standard stencil: FP32 3D four steps when the
-    // lattices give four-step tiles chunks of 32 planes or more (192^3 and
-    // up, ensembles), else three, 16-wave work-groups; FP64 3D three steps,
+    // lattices give four-step tiles chunks of 32 planes or more that divide
+    // the side (most from 192^3 up, ensembles), else three, 16-wave work-groups; FP64 3D three steps,
     // 8-wave work-groups, two rows per wave; 2D six steps (FP32 from 2^25
     // sites: eight).  Higher orders: high_order_default_depth.
     if (c->p.stencil_setting > 0)
