@@ -130,7 +130,8 @@ int ensure_pinned(Context *c, size_t bytes)
         c->pinned = nullptr;
         c->pinned_bytes = 0;
     }
-    AXS_HIP_TRY(hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault));
+    // coherent: kernels read and write it while the host fills and empties other slots
+    AXS_HIP_TRY(hipHostMalloc(&c->pinned, bytes, hipHostMallocCoherent));
     c->pinned_bytes = bytes;
     return AXS_OK;
 }
@@ -436,7 +437,7 @@ static int create_impl(const axs_params *p, int n_members, const int *Ns, axs_ct
         return fail(AXS_ERR_HIP);
     }
     const size_t mail_b = std::max<size_t>(4096, ((size_t)n_members * 16 + 255) & ~(size_t)255);
-    if (hipHostMalloc(&c->mail, mail_b + kListDirect, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&c->mail, mail_b + kListDirect, hipHostMallocCoherent) != hipSuccess) {
         set_error("pinned result buffer failed");
         return fail(AXS_ERR_OUT_OF_MEMORY);
     }
