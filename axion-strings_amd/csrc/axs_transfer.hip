@@ -1,6 +1,6 @@
 // axs_transfer.hip -- bulk transfers between the device arrays and a caller's
 // pageable arrays: host threads that (de)interleave, and the chunk pipeline
-// that keeps the copy engine and the threads busy together.
+// that keeps the link to the host and the threads busy together.
 //
 // A transfer is a list of segments (one device array each).  It is cut into
 // chunks that pass through a ring of pinned slots: to the host, a chunk is
